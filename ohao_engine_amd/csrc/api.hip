@@ -1167,12 +1167,12 @@ int render_reference(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
             launch_ref_generate(x.fl, x.pl, x.s);
         }
         // step s: the closest-hit rays queued by step s - 1 (the camera rays at s = 0)
-        // with that step's shadow rays, then shading; slot kShadowCounterBase + 63 stays 0
+        // with that step's shadow rays, then shading
         for (uint32_t st = 0; st < nsteps; ++st) {
             for (int l = 0; l < nl; ++l) {
                 const Lane& x = ln[l];
-                launch_ref_trace(S, x.pl.q[st & 1u], x.pl.counters + st, x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
-                                 x.pl.counters + kShadowCounterBase + (st ? st - 1u : 63u), st ? 2u * x.fl.n_paths : 0u,
+                launch_ref_trace(S, x.pl.q[st & 1u], x.pl.counters + ext_counter(st), x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
+                                 x.pl.counters + sh_counter(st), st ? 2u * x.fl.n_paths : 0u,
                                  x.pl.sh_o, x.pl.sh_d, x.pl.ln0, x.pl.ln1, x.pl.counters + kExtendFetchBase + st, x.ovf,
                                  x.s, tblocks);
             }
@@ -1329,8 +1329,8 @@ int ohpt_render(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
                 const Lane& x = ln[l];
                 Seg sg{};
                 if ((r = mark(&sg.a))) return r;
-                launch_extend_connect(S, x.pl.q[(b + 1) & 1u], x.pl.counters + b + 1, x.fl.n_paths, x.pl.o, x.pl.d,
-                                      x.pl.hits, x.pl.counters + kShadowCounterBase + b, 2u * x.fl.n_paths,
+                launch_extend_connect(S, x.pl.q[(b + 1) & 1u], x.pl.counters + ext_counter(b + 1), x.fl.n_paths, x.pl.o, x.pl.d,
+                                      x.pl.hits, x.pl.counters + sh_counter(b + 1), 2u * x.fl.n_paths,
                                       x.pl.sh_o, x.pl.sh_d, x.pl.sh_c, x.pl.ln0, x.pl.ln1,
                                       x.pl.counters + kExtendFetchBase + b + 1, x.ovf, nullptr, b, tstats, x.s,
                                       tblocks);
@@ -1358,8 +1358,8 @@ int ohpt_render(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
             HIPCHK(hipStreamSynchronize(c->stream));
             for (int l = 0; l < nl; ++l) {
                 const uint32_t* hc = host_counters.data() + (size_t)l * kCounterWords;
-                for (uint32_t b = 0; b <= f.max_bounces; ++b) rays_ext += hc[b];
-                for (uint32_t b = 0; b < f.max_bounces; ++b) rays_sh += hc[kShadowCounterBase + b];
+                for (uint32_t b = 0; b <= f.max_bounces; ++b) rays_ext += hc[ext_counter(b)];
+                for (uint32_t b = 0; b < f.max_bounces; ++b) rays_sh += hc[sh_counter(b + 1)];
             }
         }
         c->sample_index += batch;
@@ -1558,8 +1558,8 @@ int ohpt_adjoint(ohpt_context* c, const float* dl_dimage, int on_device, uint32_
             if (b == f.max_bounces) break;
             for (int l = 0; l < nl; ++l) {
                 const Lane& x = ln[l];
-                launch_extend_connect(S, x.pl.q[(b + 1) & 1u], x.pl.counters + b + 1, x.fl.n_paths, x.pl.o, x.pl.d,
-                                      x.pl.hits, x.pl.counters + kShadowCounterBase + b, 2u * x.fl.n_paths,
+                launch_extend_connect(S, x.pl.q[(b + 1) & 1u], x.pl.counters + ext_counter(b + 1), x.fl.n_paths, x.pl.o, x.pl.d,
+                                      x.pl.hits, x.pl.counters + sh_counter(b + 1), 2u * x.fl.n_paths,
                                       x.pl.sh_o, x.pl.sh_d, x.pl.sh_c, x.pl.ln0, x.pl.ln1,
                                       x.pl.counters + kExtendFetchBase + b + 1, x.ovf, vis, b, nullptr, x.s,
                                       tblocks);
@@ -1585,7 +1585,7 @@ int ohpt_adjoint(ohpt_context* c, const float* dl_dimage, int on_device, uint32_
             if (!retrace || b == f.max_bounces) continue;
             for (int l = 0; l < nl; ++l) {
                 const Lane& x = ln[l];
-                launch_extend(S, x.pl.q[(b + 1) & 1u], x.pl.counters + b + 1, x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
+                launch_extend(S, x.pl.q[(b + 1) & 1u], x.pl.counters + ext_counter(b + 1), x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
                               x.pl.counters + kExtendFetchBase + b + 1, x.ovf, nullptr, x.s, tblocks);
             }
         }

@@ -530,9 +530,10 @@ __device__ __forceinline__ bool ref_continue(const RefFrame& f, RefStep& P, cons
 }
 
 // Queue entry j of step `step` (j >= count: the lane only takes part in the
-// wave's appends).
+// block's appends).
 __device__ __forceinline__ void ref_shade_one(const DevScene& S, const RefFrame& f, const PathState& ps,
-                                              uint32_t step, uint32_t j, uint32_t count, const float4* srgb) {
+                                              uint32_t step, uint32_t j, uint32_t count, const float4* srgb,
+                                              uint32_t* app) {
     const uint32_t* __restrict__ qin = ps.q[step & 1u];
     uint32_t* __restrict__ qout = ps.q[(step + 1u) & 1u];
     const bool active = j < count;
@@ -631,14 +632,12 @@ __device__ __forceinline__ void ref_shade_one(const DevScene& S, const RefFrame&
             ps.ln1[pid] = P.emit_e ? P.she_c : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
     }
-    // queue appends (all lanes take part in the ballots)
-    uint32_t* cnt_sh = ps.counters + kShadowCounterBase + step;
-    const uint32_t sl = wave_append(cnt_sh, P.emit_l);
-    const uint32_t se = wave_append(cnt_sh, P.emit_e);
-    if (P.emit_l) { ps.sh_o[sl] = P.shl_o; ps.sh_d[sl] = P.shl_d; }
-    if (P.emit_e) { ps.sh_o[se] = P.she_o; ps.sh_d[se] = P.she_d; }
-    const uint32_t sn = wave_append(ps.counters + step + 1u, P.emit_next);
-    if (P.emit_next) qout[sn] = pid;
+    // queue appends (every thread of the block takes part)
+    const QueueSlots at = block_append<kRefShadeBlock / 64>(ps.counters + ext_counter(step + 1u), P.emit_next,
+                                                            P.emit_l, P.emit_e, app);
+    if (P.emit_l) { ps.sh_o[at.sh_l] = P.shl_o; ps.sh_d[at.sh_l] = P.shl_d; }
+    if (P.emit_e) { ps.sh_o[at.sh_e] = P.she_o; ps.sh_d[at.sh_e] = P.she_d; }
+    if (P.emit_next) qout[at.next] = pid;
 }
 
 // Persistent over the step's queue (its length is known only on the device):
@@ -648,7 +647,8 @@ __device__ __forceinline__ void ref_shade_one(const DevScene& S, const RefFrame&
 constexpr uint32_t kRefSrgbMax = 256;
 __global__ __launch_bounds__(kRefShadeBlock) void k_ref_shade(DevScene S, RefFrame f, PathState ps, uint32_t step) {
     __shared__ float4 srgb[kRefSrgbMax];
-    const uint32_t count = ps.counters[step];
+    __shared__ uint32_t app[2 * (kRefShadeBlock / 64) + 2];
+    const uint32_t count = ps.counters[ext_counter(step)];
     if (blockIdx.x * kRefShadeBlock >= count) return;   // uniform per block
     const bool table = S.n_materials <= kRefSrgbMax;
     if (table) {
@@ -658,8 +658,10 @@ __global__ __launch_bounds__(kRefShadeBlock) void k_ref_shade(DevScene S, RefFra
         }
         __syncthreads();
     }
-    for (uint32_t base = blockIdx.x * kRefShadeBlock; base < count; base += gridDim.x * kRefShadeBlock)
-        ref_shade_one(S, f, ps, step, base + threadIdx.x, count, table ? srgb : nullptr);
+    for (uint32_t base = blockIdx.x * kRefShadeBlock; base < count; base += gridDim.x * kRefShadeBlock) {
+        ref_shade_one(S, f, ps, step, base + threadIdx.x, count, table ? srgb : nullptr, app);
+        __syncthreads();   // app is read before the next entries' appends
+    }
 }
 
 // Per pixel, the batch's samples in sample order into the accumulation.

@@ -136,7 +136,8 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DevScene S, FrameParams f
                                                        AdjointParams adj) {
     const uint32_t* __restrict__ qin = ps.q[bounce & 1u];
     uint32_t* __restrict__ qout = ps.q[(bounce + 1u) & 1u];
-    const uint32_t count = ps.counters[bounce];
+    const uint32_t count = ps.counters[ext_counter(bounce)];
+    if (blockIdx.x * kShadeBlock >= count) return;   // whole block
     const uint32_t j = blockIdx.x * kShadeBlock + threadIdx.x;
     const bool active = j < count;
     bool emit_next = false, emit_l = false, emit_e = false;
@@ -357,16 +358,15 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DevScene S, FrameParams f
             ps.d[pid] = next_d;
         }
     }
-    // compaction (all lanes participate in the ballots)
+    // compaction (every thread of the block takes part)
+    __shared__ uint32_t app[2 * (kShadeBlock / 64) + 2];
+    const QueueSlots at = block_append<kShadeBlock / 64>(ps.counters + ext_counter(bounce + 1), emit_next, emit_l,
+                                                         emit_e, app);
     if (!kAdjoint) {
-        uint32_t* cnt_sh = ps.counters + kShadowCounterBase + bounce;
-        const uint32_t sl = wave_append(cnt_sh, emit_l);
-        const uint32_t se = wave_append(cnt_sh, emit_e);
-        if (emit_l) { ps.sh_o[sl] = shl_o; ps.sh_d[sl] = shl_d; ps.sh_c[sl] = shl_c; }
-        if (emit_e) { ps.sh_o[se] = she_o; ps.sh_d[se] = she_d; ps.sh_c[se] = she_c; }
+        if (emit_l) { ps.sh_o[at.sh_l] = shl_o; ps.sh_d[at.sh_l] = shl_d; ps.sh_c[at.sh_l] = shl_c; }
+        if (emit_e) { ps.sh_o[at.sh_e] = she_o; ps.sh_d[at.sh_e] = she_d; ps.sh_c[at.sh_e] = she_c; }
     }
-    const uint32_t sn = wave_append(ps.counters + bounce + 1, emit_next);
-    if (emit_next) qout[sn] = pid;
+    if (emit_next) qout[at.next] = pid;
 }
 
 // Deterministic gradient reduction: records sorted by key (stable, so equal

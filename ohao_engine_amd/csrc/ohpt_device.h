@@ -705,17 +705,48 @@ OHPT_DEV bool sample_analytic(const float4* L5, f3 p, float u1, float u2, f3& wi
 // ------------------------------------------------------------------ wave helpers
 OHPT_DEV uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
-// Wave-aggregated append: returns the slot for this lane (valid only when pred).
-OHPT_DEV uint32_t wave_append(uint32_t* counter, bool pred) {
-    const uint64_t mask = __ballot(pred);
-    if (mask == 0) return 0;
-    const uint32_t lo = (uint32_t)mask, hi = (uint32_t)(mask >> 32);
-    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-    const int leader = __ffsll((unsigned long long)mask) - 1;
-    uint32_t base = 0;
-    if ((int)lane_id() == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    return base + rank;
+// Queue slots of one lane's appends: its next ray and its two shadow rays
+// (each valid only when the matching predicate holds).
+struct QueueSlots {
+    uint32_t next, sh_l, sh_e;
+};
+
+// Block-aggregated append to a step's pair of queues (ext_counter, sh_counter):
+// every thread of the block calls it; `pair` counts rays in its low word and
+// shadow rays in its high word. kWaves = waves per block; lds holds
+// 2 * kWaves + 2 words, free again after the caller's next barrier.
+// The counters of a step lie on one cache line that all eight XCDs add to, and
+// these additions are taken one after another: three per wave bounded the
+// shading kernels. One per block of four waves: 1080p procedural frame 3.23 ->
+// 3.12 ms, reference estimator 5.13 -> 4.70, 256x256 Cornell frame 0.474 ->
+// 0.425, inverse-fit view (512x512, 16 samples) 20.7 -> 18.6 (blocks of 512 and
+// 1024 threads measured slower: their waves wait longer for each other).
+template <int kWaves>
+OHPT_DEV QueueSlots block_append(uint32_t* pair, bool next, bool sh_l, bool sh_e, uint32_t* lds) {
+    const uint64_t mn = __ballot(next), ml = __ballot(sh_l), me = __ballot(sh_e);
+    const uint32_t w = threadIdx.x >> 6;
+    const uint32_t nl = (uint32_t)__popcll(ml);
+    if (lane_id() == 0) {
+        lds[w] = (uint32_t)__popcll(mn);
+        lds[kWaves + w] = nl + (uint32_t)__popcll(me);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t tn = 0, ts = 0;
+        for (int k = 0; k < kWaves; ++k) { tn += lds[k]; ts += lds[kWaves + k]; }
+        unsigned long long base = 0;
+        if (tn | ts)
+            base = atomicAdd(reinterpret_cast<unsigned long long*>(pair), (unsigned long long)ts << 32 | tn);
+        lds[2 * kWaves] = (uint32_t)base;
+        lds[2 * kWaves + 1] = (uint32_t)(base >> 32);
+    }
+    __syncthreads();
+    uint32_t bn = lds[2 * kWaves], bs = lds[2 * kWaves + 1];
+    for (uint32_t k = 0; k < w; ++k) { bn += lds[k]; bs += lds[kWaves + k]; }
+    auto rank = [](uint64_t m) {
+        return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    };
+    return {bn + rank(mn), bs + rank(ml), bs + nl + rank(me)};
 }
 
 }  // namespace ohpt

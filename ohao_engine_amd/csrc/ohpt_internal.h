@@ -139,9 +139,16 @@ struct PathState {
     // then traces nothing.
     float4* hit_log;
 };
-constexpr uint32_t kShadowCounterBase = 64;       // [64 + b]: shadow rays queued at bounce b
+// Queue lengths in pairs of words, one pair per traversal step b: word 2b the
+// closest-hit rays of step b, word 2b + 1 the shadow rays that step b - 1
+// queued (traced in the same launch; word 1 stays 0). A shading step queues
+// both with one 64-bit addition (block_append).
+constexpr uint32_t ext_counter(uint32_t b) { return 2u * b; }
+constexpr uint32_t sh_counter(uint32_t b) { return 2u * b + 1u; }
 constexpr uint32_t kExtendFetchBase = 128;        // [128 + b]: dynamic-fetch counter of traversal launch b
 constexpr uint32_t kCounterWords = 192;
+// depth 60 steps to pair 61, the reference estimator's 2 + 2 * 30 steps to pair 62
+static_assert(sh_counter(62) < kExtendFetchBase && kCounterWords % 2 == 0, "counter pairs stay 8-byte aligned and clear of the fetch counters");
 
 void launch_fill_u32(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s);
 void launch_generate(const FrameParams& f, const PathState& ps, hipStream_t s);
