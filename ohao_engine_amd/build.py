@@ -20,7 +20,7 @@ LIB = PKG / "libohpt.so"
 ARCH = os.environ.get("OHPT_ARCH", "gfx950")
 
 SOURCES = ["api.hip", "lbvh.hip", "traverse.hip", "compat.hip", "integrator.hip", "env.hip", "denoiser.hip",
-           "atrous.hip"]
+           "atrous.hip", "texture.hip"]
 HEADERS = ["ohpt_device.h", "ohpt_internal.h", "ohpt_trace.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

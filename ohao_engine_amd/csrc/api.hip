@@ -48,15 +48,6 @@ struct TexStore {
     size_t packed_floats() const { return (size_t)w * h * (c >= 2 ? 4u : 1u); }
 };
 
-// Per-channel means of w*h texels with `channels` interleaved channels.
-void texel_means(const float* texels, size_t n, uint32_t channels, double mean[3]) {
-    double s[3] = {0, 0, 0};
-    for (size_t i = 0; i < n; ++i)
-        for (uint32_t k = 0; k < 3 && k < channels; ++k) s[k] += texels[i * channels + k];
-    for (int k = 0; k < 3; ++k) mean[k] = n ? s[k] / (double)n : 0.0;
-    if (channels == 1) mean[1] = mean[2] = mean[0];
-}
-
 
 }  // namespace
 
@@ -909,6 +900,33 @@ int ohpt_upload_materials(ohpt_context* c, const ohpt_material* m, uint32_t coun
     return build_emitters(c);
 }
 
+extern "C++" {
+namespace {
+// The packed texels and channel means of t from w*h*c floats. The source is first
+// copied whole, in device memory too: the copy is what checks its range, reaches
+// peers' memory and waits for the default stream's earlier work on it, while the
+// kernels stay ordered behind the context's own renders.
+int fill_texture(ohpt_context* c, TexStore& t, const float* texels, int on_device) {
+    const size_t n = (size_t)t.w * t.h, bytes = n * t.c * 4;
+    const size_t mean_at = (bytes + 15) & ~size_t(15);
+    HIPCHK(t.data.ensure(t.packed_floats() * 4));
+    HIPCHK(c->tmp.ensure(mean_at + texel_mean_scratch_bytes()));
+    if (on_device) {
+        HIPCHK(hipMemcpy(c->tmp.p, texels, bytes, hipMemcpyDefault));
+        HIPCHK(hipStreamSynchronize(nullptr));
+    } else {
+        HIPCHK(hipMemcpyAsync(c->tmp.p, texels, bytes, hipMemcpyHostToDevice, c->stream));
+    }
+    char* mean = reinterpret_cast<char*>(c->tmp.p) + mean_at;
+    launch_texel_pack(c->tmp.as<float>(), n, t.c, t.data.as<float>(), mean, c->stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(t.mean, mean, sizeof t.mean, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return OHPT_OK;
+}
+}  // namespace
+}  // extern "C++"
+
 int ohpt_upload_texture(ohpt_context* c, int32_t* out_id, const float* texels, uint32_t w, uint32_t h,
                         uint32_t channels) {
     if (!c || !out_id || !texels || w == 0 || h == 0 || channels == 0 || channels > 4)
@@ -916,16 +934,7 @@ int ohpt_upload_texture(ohpt_context* c, int32_t* out_id, const float* texels, u
     HIPCHK(enter(c));
     TexStore t;
     t.w = w; t.h = h; t.c = channels;
-    const size_t n = (size_t)w * h;
-    const uint32_t stride = channels >= 2 ? 4u : 1u;
-    std::vector<float> packed(n * stride, 0.0f);
-    for (size_t i = 0; i < n; ++i)
-        for (uint32_t k = 0; k < channels; ++k) packed[i * stride + k] = texels[i * channels + k];
-    if (channels == 3) for (size_t i = 0; i < n; ++i) packed[i * 4 + 3] = 1.0f;
-    texel_means(texels, n, channels, t.mean);
-    HIPCHK(t.data.ensure(packed.size() * 4));
-    HIPCHK(hipMemcpyAsync(t.data.p, packed.data(), packed.size() * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (int r = fill_texture(c, t, texels, 0)) return r;
     c->textures.push_back(std::move(t));
     *out_id = (int32_t)c->textures.size() - 1;
     return upload_texdesc(c);
@@ -937,21 +946,7 @@ int ohpt_update_texture(ohpt_context* c, int32_t id, const float* texels, int on
         return fail(OHPT_ERR_INVALID_ARG, "ohpt_update_texture: bad arguments");
     HIPCHK(enter(c));
     TexStore& t = c->textures[(size_t)id];
-    const size_t n = (size_t)t.w * t.h;
-    const uint32_t stride = t.c >= 2 ? 4u : 1u;
-    std::vector<float> src;
-    if (on_device) {
-        src.resize(n * t.c);
-        HIPCHK(hipMemcpy(src.data(), texels, src.size() * 4, hipMemcpyDeviceToHost));
-        texels = src.data();
-    }
-    std::vector<float> packed(n * stride, 0.0f);
-    for (size_t i = 0; i < n; ++i)
-        for (uint32_t k = 0; k < t.c; ++k) packed[i * stride + k] = texels[i * t.c + k];
-    if (t.c == 3) for (size_t i = 0; i < n; ++i) packed[i * 4 + 3] = 1.0f;
-    texel_means(texels, n, t.c, t.mean);
-    HIPCHK(hipMemcpyAsync(t.data.p, packed.data(), packed.size() * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (int r = fill_texture(c, t, texels, on_device)) return r;
     // an emissive texture's mean weighs its material's triangles in the emitter table
     for (const ohpt_material& m : c->h_materials)
         if (m.emissive_tex == id) {
@@ -1422,17 +1417,21 @@ int ohpt_read_texture_gradient(ohpt_context* c, int32_t id, float* out, int on_d
     if (!c->grad_arena.p || (size_t)id >= c->grad_off.size())
         return fail(OHPT_ERR_STATE, "ohpt_read_texture_gradient: no adjoint has run");
     HIPCHK(enter(c));
-    const size_t n = (size_t)t.w * t.h;
-    const uint32_t stride = t.c >= 2 ? 4u : 1u;
-    std::vector<float> packed(n * stride);
-    HIPCHK(hipMemcpyAsync(packed.data(), c->grad_arena.as<float>() + c->grad_off[(size_t)id], packed.size() * 4,
-                          hipMemcpyDeviceToHost, c->stream));
+    const size_t n = (size_t)t.w * t.h, bytes = n * t.c * 4;
+    const float* src = c->grad_arena.as<float>() + c->grad_off[(size_t)id];
+    if (t.c == 2 || t.c == 3) {
+        HIPCHK(c->tmp.ensure(bytes));
+        launch_texel_unpack(src, n, t.c, c->tmp.as<float>(), c->stream);
+        HIPCHK(hipGetLastError());
+        src = c->tmp.as<float>();
+    }
+    if (!on_device) HIPCHK(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    std::vector<float> dense(n * t.c);
-    for (size_t i = 0; i < n; ++i)
-        for (uint32_t k = 0; k < t.c; ++k) dense[i * t.c + k] = packed[i * stride + k];
-    if (on_device) HIPCHK(hipMemcpy(out, dense.data(), dense.size() * 4, hipMemcpyHostToDevice));
-    else std::memcpy(out, dense.data(), dense.size() * 4);
+    if (on_device) {
+        // on the default stream, behind the caller's earlier work on `out` there
+        HIPCHK(hipMemcpy(out, src, bytes, hipMemcpyDefault));
+        HIPCHK(hipStreamSynchronize(nullptr));
+    }
     return OHPT_OK;
 }
 

@@ -204,6 +204,15 @@ void launch_tonemap(const float4* accum, uint8_t* out, uint32_t n, hipStream_t s
 void launch_resolve_aovs(const float4* accum, const float4* aov_albedo, const float4* aov_normal,
                          float* albedo, float* normal, float* depth, uint32_t n, hipStream_t s);
 
+// ---- texel layout (texture.hip) ---------------------------------------------
+// n texels of `channels` floats -> the packed copy (float4 per texel, missing
+// channels 0 and a three-channel alpha 1; one float for one channel), and the mean
+// of each of the first three channels as three doubles at the start of scratch.
+size_t texel_mean_scratch_bytes();
+void launch_texel_pack(const float* src, size_t n, uint32_t channels, float* packed, void* scratch, hipStream_t s);
+// n packed float4 texels -> 2 or 3 floats each (1 and 4 channels are stored dense).
+void launch_texel_unpack(const float* packed, size_t n, uint32_t channels, float* dst, hipStream_t s);
+
 // ---- environment (env.hip) -------------------------------------------------
 // Per-row luminance*sin(theta) prefix sums, normalised, plus marginal (env_cdf.cpp:13-61).
 // Also fills the guide tables: marg_guide 2^env_guide_log2(H)+1 entries,
