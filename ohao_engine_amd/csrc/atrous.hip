@@ -21,105 +21,157 @@ namespace {
 
 constexpr float kLw[3] = {0.2126f, 0.7152f, 0.0722f};
 
-// Per-pixel records: cv = (display colour rgb, luminance variance), geo =
-// (normal xyz, depth): one 16-byte load each per filter tap.
-__global__ __launch_bounds__(256) void k_svgf_prep(const float4* __restrict__ acc, const float4* __restrict__ disp,
-                                                   const float4* __restrict__ aa, const float4* __restrict__ an,
-                                                   uint32_t n, float4* __restrict__ cv, float4* __restrict__ geo) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float cnt = acc[i].w;
-    const float4 d = disp[i], al = aa[i], nm = an[i];
-    const float inv = cnt > 0.0f ? 1.0f / cnt : 0.0f;
-    const float cx = d.x * inv, cy = d.y * inv, cz = d.z * inv;
-    const float m1 = kLw[0] * cx + kLw[1] * cy + kLw[2] * cz;
-    cv[i] = make_float4(cx, cy, cz, fmaxf(0.0f, d.w * inv - m1 * m1));
-    float nx = nm.x * inv, ny = nm.y * inv, nz = nm.z * inv;
-    const float len = sqrtf(nx * nx + ny * ny + nz * nz);
-    if (len > 0.0f) { nx /= len; ny /= len; nz /= len; }
-    const float hits = nm.w;   // samples whose primary ray hit (the AOV hit flag summed)
-    const float depth = (hits * 2.0f > cnt && hits > 0.0f) ? al.w / hits : 1e30f;
-    geo[i] = make_float4(nx, ny, nz, depth);
-}
-
 __device__ __forceinline__ float luma(float4 c) { return kLw[0] * c.x + kLw[1] * c.y + kLw[2] * c.z; }
 
-// Blocks of 64 x 4 pixels: a wave reads one row segment of 64 records per tap.
+// Blocks of 64 x 4: a wave reads one row segment of 64 records per tap.
 constexpr int kBX = 64, kBY = 4;
 
-// Short accumulations (< 4 samples): the moment variance is unreliable, so the
-// variance is at least the 3x3 luminance variance of the display image (taps
-// clamped to the edge, 9 of them), rt_svgf_temporal.comp:105-120.
-__global__ __launch_bounds__(256) void k_svgf_bootstrap(const float4* __restrict__ acc, const float4* __restrict__ cvin,
-                                                        int W, int H, float4* __restrict__ cvout) {
+// Per-pixel records: cv = (display colour rgb, luminance variance), geo =
+// (normal xyz, depth): one 16-byte load each per filter tap. While a pixel has
+// fewer than 4 samples its moment variance is unreliable, so the variance is at
+// least the 3x3 luminance variance of the display image (taps clamped to the edge,
+// 9 of them), rt_svgf_temporal.comp:105-120.
+// Bounded by HBM (96 B per pixel, the neighbours hit the caches): 1920x1080 in 41 us
+// where a record pass and a variance pass over its output took 29 + 20 us.
+__global__ __launch_bounds__(256) void k_svgf_prep(const float4* __restrict__ acc, const float4* __restrict__ disp,
+                                                   const float4* __restrict__ aa, const float4* __restrict__ an, int W,
+                                                   int H, float4* __restrict__ cv, float4* __restrict__ geo) {
     const int x = blockIdx.x * kBX + (threadIdx.x % kBX), y = blockIdx.y * kBY + (threadIdx.x / kBX);
     if (x >= W || y >= H) return;
     const int p = y * W + x;
-    float4 c = cvin[p];
-    if (acc[p].w < 4.0f) {
+    auto colour = [&](int q, float inv) {
+        const float4 d = disp[q];
+        return make_float4(d.x * inv, d.y * inv, d.z * inv, d.w * inv);
+    };
+    const float cnt = acc[p].w;
+    const float4 al = aa[p], nm = an[p];
+    const float inv = cnt > 0.0f ? 1.0f / cnt : 0.0f;
+    float4 c = colour(p, inv);
+    const float m1 = luma(c);
+    c.w = fmaxf(0.0f, c.w - m1 * m1);
+    if (cnt < 4.0f) {
         float s = 0.0f, s2 = 0.0f;
+#pragma unroll
         for (int dy = -1; dy <= 1; ++dy)
+#pragma unroll
             for (int dx = -1; dx <= 1; ++dx) {
-                const int qx = min(max(x + dx, 0), W - 1), qy = min(max(y + dy, 0), H - 1);
-                const float l = luma(cvin[qy * W + qx]);
+                const int q = min(max(y + dy, 0), H - 1) * W + min(max(x + dx, 0), W - 1);
+                const float qc = acc[q].w;
+                const float l = luma(colour(q, qc > 0.0f ? 1.0f / qc : 0.0f));
                 s += l;
                 s2 += l * l;
             }
         const float mm = s / 9.0f;
         c.w = fmaxf(c.w, fmaxf(0.0f, s2 / 9.0f - mm * mm));
     }
-    cvout[p] = c;
+    cv[p] = c;
+    float nx = nm.x * inv, ny = nm.y * inv, nz = nm.z * inv;
+    const float len = sqrtf(nx * nx + ny * ny + nz * nz);
+    if (len > 0.0f) { nx /= len; ny /= len; nz /= len; }
+    const float hits = nm.w;   // samples whose primary ray hit (the AOV hit flag summed)
+    const float depth = (hits * 2.0f > cnt && hits > 0.0f) ? al.w / hits : 1e30f;
+    geo[p] = make_float4(nx, ny, nz, depth);
 }
 
 // One iteration, rt_svgf_atrous.comp:49-115. The three edge stops are one
 // exponential of the summed exponents. The last iteration writes alpha 1.
-__global__ __launch_bounds__(256) void k_svgf_atrous(const float4* __restrict__ cvin, const float4* __restrict__ geo,
+//
+// A thread filters R pixels of its column, `step` rows apart: they share tap rows,
+// so R + 4 rows of five taps are loaded for R outputs (10 taps per pixel at R = 4
+// where one pixel per thread loads 25), and a tap's luminance is taken once. Rows
+// are uniform per wave (scalar row addresses). Bounded by vector issue, about 16
+// operations and a quarter-rate exponential per tap and output; one pixel per
+// thread was bounded by the 50 16-byte L1 reads per pixel. 1920x1080:
+// 121 us an iteration with one pixel per thread, 54 us now; the whole filter 0.64 -> 0.30 ms.
+template <int R>
+__global__ __launch_bounds__(256, 4) void k_svgf_atrous(const float4* __restrict__ cvin, const float4* __restrict__ geo,
                                                      int W, int H, int step, int last, float sigma_l, float sigma_n,
                                                      float sigma_d, float4* __restrict__ cvout) {
-    const int x = blockIdx.x * kBX + (threadIdx.x % kBX), y = blockIdx.y * kBY + (threadIdx.x / kBX);
-    if (x >= W || y >= H) return;
-    const int p = y * W + x;
-    const float4 cc = cvin[p], cg = geo[p];
-    const float cl = luma(cc);
-    // 3x3 Gaussian prefilter of the variance for the luminance edge stop (weights sum to 1)
-    const float gk[3] = {0.25f, 0.5f, 0.25f};
-    float cvar = 0.0f;
-    for (int dy = -1; dy <= 1; ++dy)
-        for (int dx = -1; dx <= 1; ++dx) {
-            const int qx = min(max(x + dx, 0), W - 1), qy = min(max(y + dy, 0), H - 1);
-            cvar += gk[dx + 1] * gk[dy + 1] * cvin[qy * W + qx].w;
+    const int x = blockIdx.x * kBX + (threadIdx.x % kBX);
+    // row group j: rows y0, y0 + step, .. of a band of R * step rows
+    const int j = __builtin_amdgcn_readfirstlane((int)(blockIdx.y * kBY + threadIdx.x / kBX));
+    const int band = j / step;
+    const int y0 = band * R * step + (j - band * step);
+    if (x >= W || y0 >= H) return;
+    const float kLog2e = 1.4426950408889634f;
+    const float inv_n = kLog2e / (sigma_n * sigma_n + 1e-4f);
+    const float inv_d = kLog2e / (sigma_d * sigma_d + 1e-4f);
+    int xq[5];
+#pragma unroll
+    for (int dx = 0; dx < 5; ++dx) xq[dx] = min(max(x + (dx - 2) * step, 0), W - 1);
+    const int xm = max(x - 1, 0), xp = min(x + 1, W - 1);
+    float4 cg[R];
+    float cl[R], cvar[R], inv_l[R];
+    float sr[R], sg[R], sb[R], ws[R], vs[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int y = min(y0 + k * step, H - 1);   // rows below the image are not written
+        cg[k] = geo[(size_t)y * W + x];
+        cl[k] = luma(cvin[(size_t)y * W + x]);
+        // 3x3 Gaussian prefilter of the variance for the luminance edge stop (weights sum to 1)
+        const float gk[3] = {0.25f, 0.5f, 0.25f};
+        float v = 0.0f;
+#pragma unroll
+        for (int dy = -1; dy <= 1; ++dy) {
+            const float4* row = cvin + (size_t)min(max(y + dy, 0), H - 1) * W;
+            v += gk[dy + 1] * (gk[0] * row[xm].w + gk[1] * row[x].w + gk[2] * row[xp].w);
         }
-    const float inv_l = 1.0f / (sqrtf(fmaxf(cvar, 1e-8f)) * sigma_l + 1e-6f);
-    const float inv_n = 1.0f / (sigma_n * sigma_n + 1e-4f);
-    const float inv_d = 1.0f / (sigma_d * sigma_d + 1e-4f);
+        cvar[k] = v;
+        inv_l[k] = kLog2e / (sqrtf(fmaxf(v, 1e-8f)) * sigma_l + 1e-6f);
+        sr[k] = sg[k] = sb[k] = ws[k] = vs[k] = 0.0f;
+    }
     const float kb[5] = {1.0f / 16.0f, 4.0f / 16.0f, 6.0f / 16.0f, 4.0f / 16.0f, 1.0f / 16.0f};
-    float sr = 0.0f, sg = 0.0f, sb = 0.0f, ws = 0.0f, vs = 0.0f;
 #pragma unroll
-    for (int dy = -2; dy <= 2; ++dy) {
-        const int qy = min(max(y + dy * step, 0), H - 1);
+    for (int m = 0; m < R + 4; ++m) {
+        int qy = min(max(y0 + (m - 2) * step, 0), H - 1);
+        // a row's loads stay behind the last row's sums: 10 records in registers, not 40
 #pragma unroll
-        for (int dx = -2; dx <= 2; ++dx) {
-            const int q = qy * W + min(max(x + dx * step, 0), W - 1);
-            const float4 sc = cvin[q], sgeo = geo[q];
-            const float nd = fmaxf(1.0f - (cg.x * sgeo.x + cg.y * sgeo.y + cg.z * sgeo.z), 0.0f);
-            const float e = fabsf(cl - luma(sc)) * inv_l + nd * inv_n + fabsf(cg.w - sgeo.w) * inv_d;
-            const float w = kb[dx + 2] * kb[dy + 2] * expf(-e);
-            sr += sc.x * w;
-            sg += sc.y * w;
-            sb += sc.z * w;
-            ws += w;
-            vs += w * w * sc.w;
+        for (int k = 0; k < R; ++k)
+            asm volatile("" : "+v"(sr[k]), "+v"(sg[k]), "+v"(sb[k]), "+v"(ws[k]), "+v"(vs[k]));
+        asm volatile("" : "+s"(qy));
+        const float4* crow = cvin + (size_t)qy * W;
+        const float4* grow = geo + (size_t)qy * W;
+#pragma unroll
+        for (int dx = 0; dx < 5; ++dx) {
+            const float4 sc = crow[xq[dx]], sgeo = grow[xq[dx]];
+            const float sl = luma(sc);
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const int dy = m - k;
+                if (dy < 0 || dy > 4) continue;
+                const float nd = fmaxf(1.0f - (cg[k].x * sgeo.x + cg[k].y * sgeo.y + cg[k].z * sgeo.z), 0.0f);
+                const float e = fabsf(cl[k] - sl) * inv_l[k] + nd * inv_n + fabsf(cg[k].w - sgeo.w) * inv_d;
+                const float w = kb[dx] * kb[dy] * __builtin_amdgcn_exp2f(-e);
+                sr[k] += sc.x * w;
+                sg[k] += sc.y * w;
+                sb[k] += sc.z * w;
+                ws[k] += w;
+                vs[k] += w * w * sc.w;
+            }
         }
     }
-    float4 o;
-    if (ws > 1e-6f) {
-        const float iw = 1.0f / ws;
-        o = make_float4(sr * iw, sg * iw, sb * iw, vs * iw * iw);
-    } else {
-        o = make_float4(cc.x, cc.y, cc.z, cvar);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int y = y0 + k * step;
+        if (y >= H) break;
+        float4 o;
+        if (ws[k] > 1e-6f) {
+            const float iw = 1.0f / ws[k];
+            o = make_float4(sr[k] * iw, sg[k] * iw, sb[k] * iw, vs[k] * iw * iw);
+        } else {
+            const float4 cc = cvin[(size_t)y * W + x];
+            o = make_float4(cc.x, cc.y, cc.z, cvar[k]);
+        }
+        if (last) o.w = 1.0f;
+        cvout[(size_t)y * W + x] = o;
     }
-    if (last) o.w = 1.0f;
-    cvout[p] = o;
+}
+
+template <int R>
+void launch_atrous(const float4* ci, const float4* geo, int W, int H, int step, int last, float4* co, hipStream_t s) {
+    const int groups = (H + R * step - 1) / (R * step) * step;
+    const dim3 grid((W + kBX - 1) / kBX, (groups + kBY - 1) / kBY);
+    k_svgf_atrous<R><<<grid, 256, 0, s>>>(ci, geo, W, H, step, last, kSvgfSigmaL, kSvgfSigmaN, kSvgfSigmaD, co);
 }
 
 }  // namespace
@@ -130,23 +182,25 @@ hipError_t svgf_atrous(const float4* accum, const float4* disp, const float4* ao
     const uint32_t n = W * H;
     if (n == 0) return hipSuccess;
     float4* c0 = reinterpret_cast<float4*>(scratch);
-    float4* c1 = c0 + n;
-    float4* geo = c1 + n;
-    k_svgf_prep<<<(n + 255) / 256, 256, 0, s>>>(accum, disp, aov_albedo, aov_normal, n, c0, geo);
+    float4* geo = c0 + n;
     const dim3 grid((W + kBX - 1) / kBX, (H + kBY - 1) / kBY);
-    k_svgf_bootstrap<<<grid, 256, 0, s>>>(accum, c0, (int)W, (int)H, c1);
-    // ping-pong c1 -> out -> c0 -> out -> c0 -> out: the odd count of 5 ends in `out`
+    k_svgf_prep<<<grid, 256, 0, s>>>(accum, disp, aov_albedo, aov_normal, (int)W, (int)H, c0, geo);
+    // ping-pong c0 -> out -> c0 -> out -> c0 -> out: the odd count of 5 ends in `out`
     static_assert(kSvgfIterations % 2 == 1, "the ping-pong below ends in `out` for an odd count");
-    const float4* ci = c1;
+    // Four pixels per thread leave small images with too few waves and a longer chain per
+    // thread: whole filter with one / four, 320x200 46 / 78 us, 512x512 73 / 79 us,
+    // 800x600 123 / 117 us, 1920x1080 390 / 301 us.
+    const bool wide = n >= 400000;
     for (int it = 0; it < kSvgfIterations; ++it) {
+        const float4* ci = (it % 2 == 0) ? c0 : out;
         float4* co = (it % 2 == 0) ? out : c0;
-        k_svgf_atrous<<<grid, 256, 0, s>>>(ci, geo, (int)W, (int)H, 1 << it, it == kSvgfIterations - 1 ? 1 : 0,
-                                           kSvgfSigmaL, kSvgfSigmaN, kSvgfSigmaD, co);
-        ci = co;
+        const int last = it == kSvgfIterations - 1 ? 1 : 0;
+        if (wide) launch_atrous<4>(ci, geo, (int)W, (int)H, 1 << it, last, co, s);
+        else launch_atrous<1>(ci, geo, (int)W, (int)H, 1 << it, last, co, s);
     }
     return hipGetLastError();
 }
 
-size_t svgf_scratch_bytes(uint32_t W, uint32_t H) { return (size_t)W * H * 48; }
+size_t svgf_scratch_bytes(uint32_t W, uint32_t H) { return (size_t)W * H * 32; }
 
 }  // namespace ohpt
