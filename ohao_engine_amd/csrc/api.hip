@@ -119,7 +119,7 @@ struct ohpt_context {
     // path state
     uint32_t capacity = 0;
     DevBuf ps_o, ps_d, ps_T, ps_L, ps_ln0, ps_ln1, ps_aov0, ps_aov1, ps_q0, ps_q1, ps_hits, sh_o, sh_d, sh_c,
-        counters, ovf, tmp, tstats;
+        counters, fetch, ovf, tmp, tstats;
     uint32_t ovf_rays = 0;
     DevBuf adj_vis, adj_lrem, adj_dldi, adj_hits;   // path-replay adjoint state
     DevBuf rec_key2, rec_val2, rec_count, rec_tiles; // deterministic mode: compacted records
@@ -242,6 +242,14 @@ int need_guides(const ohpt_context* c, const char* what) {
     return OHPT_OK;
 }
 
+// Stack overflow slots and fetch counters of the traversals, for every lane: one size
+// for the context's life, so they are never replaced under a launch in flight.
+hipError_t ensure_trace_scratch(ohpt_context* c) {
+    const hipError_t e = c->ovf.ensure(trace_overflow_bytes() * ohpt_context::kLanes);
+    return e != hipSuccess ? e
+                           : c->fetch.ensure((size_t)kFetchWords * kMaxTraceLaunches * 4 * ohpt_context::kLanes);
+}
+
 int ensure_paths(ohpt_context* c, uint32_t n) {
     if (n <= c->capacity) return OHPT_OK;
     // the buffers are replaced: nothing in flight may still use them
@@ -265,7 +273,7 @@ int ensure_paths(ohpt_context* c, uint32_t n) {
     HIPCHK(c->sh_d.ensure(2 * N * 16));
     HIPCHK(c->sh_c.ensure(2 * N * 16));
     HIPCHK(c->counters.ensure((size_t)kCounterWords * 4 * ohpt_context::kLanes));
-    HIPCHK(c->ovf.ensure(trace_overflow_bytes() * ohpt_context::kLanes));
+    HIPCHK(ensure_trace_scratch(c));
     c->ovf_rays = 2 * n;
     c->capacity = n;
     return OHPT_OK;
@@ -283,6 +291,7 @@ PathState lane_view(const PathState& ps, uint32_t pid_base, int lane) {
     p.sh_d = ps.sh_d + 2 * (size_t)pid_base;
     p.sh_c = ps.sh_c + 2 * (size_t)pid_base;
     p.counters = ps.counters + (size_t)lane * kCounterWords;
+    p.fetch = ps.fetch + (size_t)lane * kMaxTraceLaunches * kFetchWords;
     return p;
 }
 
@@ -309,6 +318,7 @@ PathState path_state(ohpt_context* c, int set = 0) {
     p.sh_d = c->sh_d.as<float4>();
     p.sh_c = c->sh_c.as<float4>();
     p.counters = c->counters.as<uint32_t>();
+    p.fetch = c->fetch.as<uint32_t>();
     p.capacity = c->capacity;
     return p;
 }
@@ -498,13 +508,13 @@ int upload_texdesc(ohpt_context* c) {
 
 // ---- scratch of the no-allocation ray query (ohpt_trace_rays_noalloc) ------
 // One array per device, in the code object: the traversal's dynamic-fetch
-// counter (first 256 bytes) and the per-thread stack-overflow slots of a
-// persistent grid of kNoAllocBlocks blocks (32 MiB + 256 B). Host code never
+// counters (first 8 KiB) and the per-thread stack-overflow slots of a
+// persistent grid of kNoAllocBlocks blocks (36 MiB + 8 KiB). Host code never
 // uses the array's name as an address: ohpt_create resolves each device's
 // copy with hipGetSymbolAddress once, and the kernels receive that pointer.
 constexpr uint32_t kNoAllocBlocks = 1024;
 constexpr size_t kNoAllocOvfBytes = (size_t)kNoAllocBlocks * kTraceBlock * kStackOvf * 4;
-constexpr size_t kNoAllocScratchBytes = 256 + kNoAllocOvfBytes;
+constexpr size_t kNoAllocScratchBytes = kFetchWords * 4 + kNoAllocOvfBytes;
 constexpr uint32_t kNoAllocMaxRays = 1u << 31;   // keeps the 32-bit fetch counter from wrapping
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
@@ -1158,7 +1168,7 @@ int render_reference(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
             x.fl.n_paths = std::min<uint32_t>(f.n_paths - x.fl.pid_base, part);
             x.pl = lane_view(ps, x.fl.pid_base, l);
             x.ovf = lane_ovf(c, l);
-            launch_fill_u32(x.pl.counters, 0u, kCounterWords, x.s);
+            launch_clear_counters(x.pl, nsteps, x.s);
             launch_ref_generate(x.fl, x.pl, x.s);
         }
         // step s: the closest-hit rays queued by step s - 1 (the camera rays at s = 0)
@@ -1168,7 +1178,7 @@ int render_reference(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
                 const Lane& x = ln[l];
                 launch_ref_trace(S, x.pl.q[st & 1u], x.pl.counters + ext_counter(st), x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
                                  x.pl.counters + sh_counter(st), st ? 2u * x.fl.n_paths : 0u,
-                                 x.pl.sh_o, x.pl.sh_d, x.pl.ln0, x.pl.ln1, x.pl.counters + kExtendFetchBase + st, x.ovf,
+                                 x.pl.sh_o, x.pl.sh_d, x.pl.ln0, x.pl.ln1, fetch_counters(x.pl, st), x.ovf,
                                  x.s, tblocks);
             }
             for (int l = 0; l < nl; ++l) launch_ref_shade(S, ln[l].fl, ln[l].pl, st, ln[l].s);
@@ -1293,7 +1303,7 @@ int ohpt_render(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
             x.fl.n_paths = std::min<uint32_t>(f.n_paths - x.fl.pid_base, part);
             x.pl = lane_view(ps, x.fl.pid_base, l);
             x.ovf = lane_ovf(c, l);
-            launch_fill_u32(x.pl.counters, 0u, kCounterWords, x.s);
+            launch_clear_counters(x.pl, f.max_bounces + 1, x.s);
             launch_generate(x.fl, x.pl, x.s);
         }
         // The lanes' kernels are submitted step by step (every lane's extend, then every
@@ -1305,7 +1315,7 @@ int ohpt_render(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
             Seg sg{};
             if ((r = mark(&sg.a))) return r;
             launch_extend(S, x.pl.q[0], x.pl.counters, x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
-                          x.pl.counters + kExtendFetchBase, x.ovf, tstats, x.s, tblocks);
+                          fetch_counters(x.pl, 0), x.ovf, tstats, x.s, tblocks);
             ++n_extend;
             if ((r = mark(&sg.b))) return r;
             if (profile) { sg.kind = 0; segs.push_back(sg); }
@@ -1327,7 +1337,7 @@ int ohpt_render(ohpt_context* c, uint32_t spp, uint32_t render_flags) {
                 launch_extend_connect(S, x.pl.q[(b + 1) & 1u], x.pl.counters + ext_counter(b + 1), x.fl.n_paths, x.pl.o, x.pl.d,
                                       x.pl.hits, x.pl.counters + sh_counter(b + 1), 2u * x.fl.n_paths,
                                       x.pl.sh_o, x.pl.sh_d, x.pl.sh_c, x.pl.ln0, x.pl.ln1,
-                                      x.pl.counters + kExtendFetchBase + b + 1, x.ovf, nullptr, b, tstats, x.s,
+                                      fetch_counters(x.pl, b + 1), x.ovf, nullptr, b, tstats, x.s,
                                       tblocks);
                 ++n_extend;
                 if ((r = mark(&sg.b))) return r;
@@ -1543,14 +1553,14 @@ int ohpt_adjoint(ohpt_context* c, const float* dl_dimage, int on_device, uint32_
             x.pl = lane_view(ps, x.fl.pid_base, l);
             x.ovf = lane_ovf(c, l);
             // pass 1: forward, recording shadow visibility
-            launch_fill_u32(x.pl.counters, 0u, kCounterWords, x.s);
+            launch_clear_counters(x.pl, f.max_bounces + 1, x.s);
             launch_fill_u32(vis + x.fl.pid_base, 0u, x.fl.n_paths, x.s);
             launch_generate(x.fl, x.pl, x.s);
         }
         for (int l = 0; l < nl; ++l) {
             const Lane& x = ln[l];
             launch_extend(S, x.pl.q[0], x.pl.counters, x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
-                          x.pl.counters + kExtendFetchBase, x.ovf, nullptr, x.s, tblocks);
+                          fetch_counters(x.pl, 0), x.ovf, nullptr, x.s, tblocks);
         }
         for (uint32_t b = 0; b <= f.max_bounces; ++b) {
             for (int l = 0; l < nl; ++l) launch_shade(S, ln[l].fl, ln[l].pl, b, ln[l].s);
@@ -1560,7 +1570,7 @@ int ohpt_adjoint(ohpt_context* c, const float* dl_dimage, int on_device, uint32_
                 launch_extend_connect(S, x.pl.q[(b + 1) & 1u], x.pl.counters + ext_counter(b + 1), x.fl.n_paths, x.pl.o, x.pl.d,
                                       x.pl.hits, x.pl.counters + sh_counter(b + 1), 2u * x.fl.n_paths,
                                       x.pl.sh_o, x.pl.sh_d, x.pl.sh_c, x.pl.ln0, x.pl.ln1,
-                                      x.pl.counters + kExtendFetchBase + b + 1, x.ovf, vis, b, nullptr, x.s,
+                                      fetch_counters(x.pl, b + 1), x.ovf, vis, b, nullptr, x.s,
                                       tblocks);
             }
         }
@@ -1571,11 +1581,11 @@ int ohpt_adjoint(ohpt_context* c, const float* dl_dimage, int on_device, uint32_
         for (int l = 0; l < nl; ++l) {
             const Lane& x = ln[l];
             launch_adjoint_init(x.pl, x.fl.pid_base, x.fl.n_paths, lrem, x.s);
-            launch_fill_u32(x.pl.counters, 0u, kCounterWords, x.s);
+            launch_clear_counters(x.pl, f.max_bounces + 1, x.s);
             launch_generate(x.fl, x.pl, x.s);
             if (retrace)
                 launch_extend(S, x.pl.q[0], x.pl.counters, x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
-                              x.pl.counters + kExtendFetchBase, x.ovf, nullptr, x.s, tblocks);
+                              fetch_counters(x.pl, 0), x.ovf, nullptr, x.s, tblocks);
         }
         for (uint32_t b = 0; b <= f.max_bounces; ++b) {
             for (int l = 0; l < nl; ++l)
@@ -1585,7 +1595,7 @@ int ohpt_adjoint(ohpt_context* c, const float* dl_dimage, int on_device, uint32_
             for (int l = 0; l < nl; ++l) {
                 const Lane& x = ln[l];
                 launch_extend(S, x.pl.q[(b + 1) & 1u], x.pl.counters + ext_counter(b + 1), x.fl.n_paths, x.pl.o, x.pl.d, x.pl.hits,
-                              x.pl.counters + kExtendFetchBase + b + 1, x.ovf, nullptr, x.s, tblocks);
+                              fetch_counters(x.pl, b + 1), x.ovf, nullptr, x.s, tblocks);
             }
         }
         if (nl > 1) {
@@ -1777,9 +1787,8 @@ int ray_batch(ohpt_context* c, const float* rays, void* out, uint32_t n, int on_
     if (int r0 = need_tree(c, "ray batch")) return r0;
     if (n == 0) return OHPT_OK;
     HIPCHK(enter(c));
-    DevBuf dr, dout, dovf, dfetch;
-    HIPCHK(dovf.ensure(trace_overflow_bytes()));
-    HIPCHK(dfetch.ensure(256));
+    DevBuf dr, dout;
+    HIPCHK(ensure_trace_scratch(c));
     const float4* r = reinterpret_cast<const float4*>(rays);
     void* o = out;
     const size_t out_bytes = (size_t)n * (occl ? 4 : 16);
@@ -1791,8 +1800,10 @@ int ray_batch(ohpt_context* c, const float* rays, void* out, uint32_t n, int on_
         o = dout.p;
     }
     const DevScene S = scene_view(c);
-    if (occl) launch_occluded_rays(S, r, reinterpret_cast<uint32_t*>(o), n, dfetch.as<uint32_t>(), dovf.as<uint32_t>(), c->stream);
-    else launch_trace_rays(S, r, reinterpret_cast<float4*>(o), n, dfetch.as<uint32_t>(), dovf.as<uint32_t>(), c->stream);
+    uint32_t* const fetch = c->fetch.as<uint32_t>();
+    uint32_t* const ovf = c->ovf.as<uint32_t>();
+    if (occl) launch_occluded_rays(S, r, reinterpret_cast<uint32_t*>(o), n, fetch, ovf, c->stream);
+    else launch_trace_rays(S, r, reinterpret_cast<float4*>(o), n, fetch, ovf, c->stream);
     HIPCHK(hipGetLastError());
     if (!on_device) HIPCHK(hipMemcpyAsync(out, dout.p, out_bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1823,8 +1834,8 @@ int ohpt_trace_rays_noalloc(ohpt_context* c, const float* rays, float* hits, uin
     HIPCHK(enter(c));
     unsigned char* base = static_cast<unsigned char*>(noalloc_scratch(c->device));
     if (!base) return fail(OHPT_ERR_STATE, "ohpt_trace_rays_noalloc: scratch not resolved for this device");
-    uint32_t* fetch = reinterpret_cast<uint32_t*>(base);          // zeroed by a kernel at launch
-    uint32_t* ovf = reinterpret_cast<uint32_t*>(base + 256);
+    uint32_t* fetch = reinterpret_cast<uint32_t*>(base);          // kFetchWords, zeroed by a kernel at launch
+    uint32_t* ovf = reinterpret_cast<uint32_t*>(base + kFetchWords * 4);
     launch_trace_rays(scene_view(c), reinterpret_cast<const float4*>(rays), reinterpret_cast<float4*>(hits), n,
                       fetch, ovf, c->stream, kNoAllocBlocks);
     HIPCHK(hipGetLastError());

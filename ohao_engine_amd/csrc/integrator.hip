@@ -29,6 +29,12 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint32_t n) {
     if (i < n) p[i] = v;
 }
 
+__global__ __launch_bounds__(256) void k_clear_counters(uint32_t* counters, uint32_t* fetch, uint32_t nfetch) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < kCounterWords) counters[i] = 0u;
+    if (i < nfetch) fetch[i] = 0u;
+}
+
 __device__ __forceinline__ f3 camera_dir(const FrameParams& f, uint32_t px, uint32_t py, float jx, float jy) {
     const float ndcx = ((float)px + 0.5f + jx) / (float)f.width * 2.0f - 1.0f;
     const float ndcy = ((float)py + 0.5f + jy) / (float)f.height * 2.0f - 1.0f;
@@ -557,6 +563,11 @@ inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) /
 
 void launch_fill_u32(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s) {
     if (n) k_fill_u32<<<div_up(n, 256), 256, 0, s>>>(p, v, n);
+}
+
+void launch_clear_counters(const PathState& ps, uint32_t launches, hipStream_t s) {
+    const uint32_t n = launches * kFetchWords;
+    k_clear_counters<<<div_up(std::max(n, kCounterWords), 256), 256, 0, s>>>(ps.counters, ps.fetch, n);
 }
 
 void launch_generate(const FrameParams& f, const PathState& ps, hipStream_t s) {

@@ -63,16 +63,23 @@ hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, uint32_t
 #define OHPT_TRACE_BLOCK 128
 #endif
 #ifndef OHPT_STACK_LDS
-#define OHPT_STACK_LDS 24   // 12 KB per block: 10 blocks (VGPR-bound 5 waves/SIMD) fit a CU's 160 KB with room to spare
+#define OHPT_STACK_LDS 16   // with the leaf queue 16 KB per block: the VGPR-bound 5 waves per SIMD (10 blocks) fill a CU's 160 KB
 #endif
 constexpr uint32_t kTraceBlock = OHPT_TRACE_BLOCK;
 constexpr uint32_t kStackLds = OHPT_STACK_LDS;   // per-thread LDS stack entries
-constexpr uint32_t kStackOvf = 64;               // per-thread global overflow entries
+constexpr uint32_t kStackOvf = 72;               // per-thread global overflow entries
 constexpr uint32_t kMaxTreeDepth = 60;   // commit rejects deeper trees (binary leaf depth, root = 1)
-// at most three pushes per 4-wide level, and a binary tree of leaf depth D has
-// at most D/2 levels of 4-wide nodes: registers (4) + LDS + overflow cover that
-static_assert(4 + kStackLds + kStackOvf >= 3 * (kMaxTreeDepth / 2), "traversal stack shallower than the deepest tree");
+// a binary tree of leaf depth D has at most D/2 levels of 4-wide nodes; each but the
+// last (its children are leaves) leaves at most three entries behind, and the four of the
+// deepest one are on the stack before the nearest is taken off
+static_assert(kStackLds + kStackOvf >= 3 * (kMaxTreeDepth / 2 - 1) + 1, "traversal stack shallower than the deepest tree");
 static_assert(kTraceBlock % 64 == 0 && kTraceBlock <= 1024, "trace block must be whole waves");
+
+// Dynamic ray fetching: one counter per group of blocks, each in a cache line of its own.
+constexpr uint32_t kFetchGroups = 64;
+constexpr uint32_t kFetchStride = 32;                          // words from one counter to the next
+constexpr uint32_t kFetchWords = kFetchGroups * kFetchStride;  // counters of one launch
+static_assert(kFetchWords % 256 == 0, "cleared in blocks of 256 words");
 
 // Persistent-thread grid of the traversal kernels and the size of their
 // global stack-overflow buffer (one kStackOvf slot per resident thread).
@@ -80,7 +87,7 @@ uint32_t trace_grid_blocks();
 size_t trace_overflow_bytes();
 
 // Closest hit for queued paths: ray of path queue[j] -> hits[j] = (t, slot|miss, u, v).
-// `fetch` is a zeroed counter used for dynamic ray fetching. max_blocks != 0 caps
+// `fetch` are kFetchWords zeroed words for dynamic ray fetching. max_blocks != 0 caps
 // the persistent grid (launches of concurrent lanes share the GPU).
 void launch_extend(const DevScene& S, const uint32_t* queue, const uint32_t* count, uint32_t max_count,
                    const float4* ray_o, const float4* ray_d, float4* hits, uint32_t* fetch, uint32_t* ovf,
@@ -132,7 +139,8 @@ struct PathState {
     float4* sh_o;
     float4* sh_d;
     float4* sh_c;
-    uint32_t* counters;   // kCounterWords: extend counts, shadow counts, fetch counters
+    uint32_t* counters;   // kCounterWords: extend counts, shadow counts
+    uint32_t* fetch;      // kFetchWords per traversal launch: dynamic-fetch counters
     uint32_t capacity;
     // Adjoint only (null otherwise): closest hit of every path vertex, written by the
     // forward pass at [bounce * capacity + pid] and read back by the replay, which
@@ -145,11 +153,15 @@ struct PathState {
 // both with one 64-bit addition (block_append).
 constexpr uint32_t ext_counter(uint32_t b) { return 2u * b; }
 constexpr uint32_t sh_counter(uint32_t b) { return 2u * b + 1u; }
-constexpr uint32_t kExtendFetchBase = 128;        // [128 + b]: dynamic-fetch counter of traversal launch b
-constexpr uint32_t kCounterWords = 192;
+constexpr uint32_t kCounterWords = 128;
+constexpr uint32_t kMaxTraceLaunches = 64;        // traversal launches of one batch
 // depth 60 steps to pair 61, the reference estimator's 2 + 2 * 30 steps to pair 62
-static_assert(sh_counter(62) < kExtendFetchBase && kCounterWords % 2 == 0, "counter pairs stay 8-byte aligned and clear of the fetch counters");
+static_assert(sh_counter(62) < kCounterWords && kCounterWords % 2 == 0, "counter pairs stay 8-byte aligned and inside their words");
 
+// The dynamic-fetch counters of traversal launch b of a batch.
+inline uint32_t* fetch_counters(const PathState& ps, uint32_t b) { return ps.fetch + (size_t)b * kFetchWords; }
+// Zeroes the queue lengths and the fetch counters of the batch's first `launches` traversals.
+void launch_clear_counters(const PathState& ps, uint32_t launches, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s);
 void launch_generate(const FrameParams& f, const PathState& ps, hipStream_t s);
 void launch_shade(const DevScene& S, const FrameParams& f, const PathState& ps, uint32_t bounce, hipStream_t s);

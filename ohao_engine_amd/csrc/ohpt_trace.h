@@ -1,5 +1,5 @@
-// Ray/box and ray/triangle tests, child ordering and the short stack of the
-// LBVH traversal (traverse.hip's persistent kernels).
+// Ray/box and ray/triangle tests and the child ordering of the LBVH traversal
+// (traverse.hip's persistent kernels).
 //
 // Ray/box: robust slab test with tmax scaled by 1+2*gamma(3) (Ize 2013).
 // Ray/triangle: watertight test of Woop, Benthin & Wald (JCGT 2013); an edge
@@ -118,40 +118,9 @@ __device__ __forceinline__ uint32_t order_key(float e, uint32_t slot) {
     const uint32_t m = (b & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u;
     return ((b ^ m) & ~3u) | slot;
 }
-__device__ __forceinline__ void cx(uint32_t& a, uint32_t& b) {
-    const uint32_t lo = min(a, b), hi = max(a, b);
-    a = lo;
-    b = hi;
-}
-
-// Register/LDS/global short stack.
-struct Stack {
-    uint32_t r0, r1, r2, r3;
-    int nreg;     // entries held in registers (top of stack)
-    int nmem;     // entries below them (LDS, then overflow)
-    __device__ __forceinline__ void reset() { nreg = 0; nmem = 0; }
-    __device__ __forceinline__ void push(uint32_t x, uint32_t* lds, uint32_t* ovf) {
-        if (nreg == 4) {
-            if (nmem < (int)kStackLds) lds[nmem * kTraceBlock] = r3;
-            else ovf[nmem - (int)kStackLds] = r3;
-            ++nmem;
-            --nreg;
-        }
-        r3 = r2; r2 = r1; r1 = r0; r0 = x;
-        ++nreg;
-    }
-    __device__ __forceinline__ bool empty() const { return nreg == 0 && nmem == 0; }
-    __device__ __forceinline__ uint32_t pop(const uint32_t* lds, const uint32_t* ovf) {
-        if (nreg > 0) {
-            const uint32_t x = r0;
-            r0 = r1; r1 = r2; r2 = r3;
-            --nreg;
-            return x;
-        }
-        --nmem;
-        return nmem < (int)kStackLds ? lds[nmem * kTraceBlock] : ovf[nmem - (int)kStackLds];
-    }
-};
+// The same order where no entry distance is negative (tmin >= +0: the maximum with
+// +0 is never -0).
+__device__ __forceinline__ uint32_t order_key_pos(float e, uint32_t slot) { return (__float_as_uint(e) & ~3u) | slot; }
 
 }  // namespace trace
 }  // namespace ohpt

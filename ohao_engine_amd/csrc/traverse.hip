@@ -6,20 +6,30 @@
 // fetching, Aila & Laine 2009) — so lanes do not wait for the longest ray of a
 // batch and no blocks are launched for rays that do not exist.
 //
-// Short-stack traversal of the 128-byte 4-wide nodes (the binary LBVH
-// collapsed two levels per node, halving the chain of dependent node fetches
-// per ray; one node is one 128-byte cache line): the top four stack entries
-// live in VGPRs (shifted on push/pop), deeper entries spill to a per-thread
-// column of LDS ([depth][thread], bank-conflict free), and beyond that to a
-// per-thread slot in global memory. At each node the hit children are ordered
-// by entry distance (order_key); hit leaves (one triangle each) are intersected in
-// that order, then the internal children whose entry is still within the
-// closest hit continue, nearest first. The visiting order and every FP
-// operation match the sequential restatement in the oracle, so hits agree bit
-// for bit.
+// Stack traversal of the 128-byte 4-wide nodes (the binary LBVH collapsed two
+// levels per node, halving the chain of dependent node fetches per ray; one node
+// is one 128-byte cache line). The stack is a per-thread column of LDS
+// ([depth][thread], bank-conflict free), deeper entries go to a per-thread slot
+// in global memory. Hit leaves (one triangle each) wait in a small queue per lane,
+// in the order of their entry distance (order_key); internal children go on the
+// stack, the nearest on top. A wave intersects queued leaves when three eighths of
+// its busy lanes have some: a ray has one leaf hit per ten node steps, so testing at once
+// ran the triangle test for a few lanes of 64 in nearly every step. The triangles
+// are tested in the order in which a sequential traversal meets them, and a leaf
+// whose entry lies behind the closest hit by then is dropped, as that traversal
+// would have: an entry distance never decreases from a node to its children, so
+// what the late hit lets through meanwhile is dropped too. Every FP operation
+// matches the sequential restatement in the oracle, and hits agree bit for bit.
 //
-// The ray/box and ray/triangle tests, the child order key and the stack are in
-// ohpt_trace.h.
+// Bounded by the vector pipe and the return of divergent node loads together (each
+// 60-70 % busy on 10^6 incoherent rays), and by the longest rays at the end of a
+// launch. Against one triangle test per leaf in the step, a sorting network with
+// selects, and one fetch counter: 10^6 rays on the 3.1M-triangle scene 541 -> 508 us,
+// its 1920x1080 frame 3.04 -> 2.74 ms, the reference estimator's frame on 2058
+// triangles 4.32 -> 3.08 ms (nearly all of it the counters'), 512x512 turntable
+// 2.41 -> 2.33 ms.
+//
+// The ray/box and ray/triangle tests and the child order key are in ohpt_trace.h.
 #pragma clang fp contract(off)
 
 #include "ohpt_trace.h"
@@ -29,14 +39,22 @@ namespace {
 
 using namespace trace;
 
-// lanes keep stepping without refilling while at least this many are busy
+// Lanes keep stepping without refilling while at least this many are busy (10^6 rays:
+// 531 us a call at 16, 517 at 24, 506 at 32, 500 at 40; turntable 2.36, 2.35, 2.32, 2.33 ms).
 #ifndef OHPT_REFILL_THRESHOLD
-#define OHPT_REFILL_THRESHOLD 16
+#define OHPT_REFILL_THRESHOLD 32
 #endif
 constexpr int kRefillThreshold = OHPT_REFILL_THRESHOLD;
 
+// Queued leaves are intersected once kDrainAt eighths of the busy lanes have some, until
+// fewer than kDrainTo eighths do (3 / 2, 4 / 3 and 3 / 1 within 1 %, 2 / 1 slower by 1 %).
+constexpr uint32_t kDrainAt = 3, kDrainTo = 2;
+constexpr uint32_t kPend = 8;   // entries per lane, a power of two of at least 4
+static_assert(kPend >= 4 && (kPend & (kPend - 1)) == 0, "a node step can queue four leaves");
+
 // Ray sources/sinks of the four kernels.
 struct ExtendIO {
+    static constexpr bool kPosTmin = true;
     const uint32_t* queue;
     const float4* ray_o;
     const float4* ray_d;
@@ -53,6 +71,7 @@ struct ExtendIO {
 };
 
 struct ConnectIO {
+    static constexpr bool kPosTmin = true;
     const float4* sh_o;
     const float4* sh_d;
     const float4* sh_c;
@@ -81,6 +100,7 @@ struct ConnectIO {
 };
 
 struct RaysIO {
+    static constexpr bool kPosTmin = false;
     const float4* rays;
     float4* hits;
     uint32_t* occl;
@@ -143,6 +163,7 @@ struct RefConnectIO {
 };
 
 struct RefFusedIO {
+    static constexpr bool kPosTmin = true;
     RefExtendIO ext;
     RefConnectIO con;
     uint32_t n_ext;
@@ -161,6 +182,7 @@ struct RefFusedIO {
 // Extension rays of one bounce and shadow rays of the previous one, traced by
 // one launch: indices [0, n_ext) are closest-hit rays, the rest any-hit.
 struct FusedIO {
+    static constexpr bool kPosTmin = true;
     ExtendIO ext;
     ConnectIO con;
     uint32_t n_ext;
@@ -179,24 +201,28 @@ struct FusedIO {
 // launches only; the counters cost registers).
 template <int kMode, bool kStats, class IO>
 __device__ __forceinline__ void persistent_trace(const DevScene& S, const IO& io, uint32_t count,
-                                                 uint32_t* __restrict__ fetch, uint32_t* lds_col, uint32_t* ovf,
-                                                 unsigned long long* stats) {
+                                                 uint32_t* fetch, uint32_t* lds_col, uint2* pend,
+                                                 uint32_t* ovf, unsigned long long* stats) {
     const uint32_t lane = lane_id();
     RayPre r;
-    Stack st;
-    st.r0 = st.r1 = st.r2 = st.r3 = 0;
-    st.reset();
-    uint32_t cur = 0, j = 0;
+    uint32_t cur = 0, j = 0, sp = 0;
     // closest hit so far: distance tclose (tmax while none), slot hprim, barycentrics hu, hv
     float tmin = 0.0f, tclose = 0.0f, hu = 0.0f, hv = 0.0f;
     uint32_t hprim = kMiss;
+    float tgroup = 0.0f;           // tclose when the first leaf of the tested one's node came up
     bool active = false, anyhit = kMode == 1;
+    bool fin = false;              // nothing left to visit; the queued leaves remain
+    uint32_t qh = 0, qn = 0;       // queued leaves: first entry, count
     uint32_t nv = 0, nt = 0;
-    // The first ray of every thread is its global index (no atomics: launches
-    // with fewer rays than resident threads never touch the counter); the
-    // shared counter hands out the rays beyond the grid.
+    // The first ray of every thread is its global index (no atomics: launches with
+    // fewer rays than resident threads never touch the counters). The rays beyond
+    // are dealt in runs of 64 to `groups` groups of blocks, each with a counter of its
+    // own in its own cache line: with one counter every wave's additions queued at one
+    // address (the reference estimator's 1080p frame 4.36 ms, 3.08 ms with 64).
     const uint32_t nthreads = gridDim.x * blockDim.x;
     bool drained = nthreads >= count;
+    const uint32_t groups = min(kFetchGroups, gridDim.x), group = blockIdx.x % groups;
+    fetch += group * kFetchStride;
     auto start = [&](uint32_t idx) {
         float3 o, d;
         float tmax;
@@ -208,7 +234,9 @@ __device__ __forceinline__ void persistent_trace(const DevScene& S, const IO& io
         hprim = kMiss;
         hu = hv = 0.0f;
         cur = 0;
-        st.reset();
+        sp = 0;
+        fin = false;
+        qn = 0;
         active = S.n_tris > 0;
         if (!active) io.store(S, j, make_float4(tclose, __uint_as_float(hprim), hu, hv));
     };
@@ -222,14 +250,15 @@ __device__ __forceinline__ void persistent_trace(const DevScene& S, const IO& io
             const uint64_t want = __ballot(!active);
             if (want != 0) {
                 const int leader = __ffsll((unsigned long long)want) - 1;
-                const uint32_t nw = (uint32_t)__popcll(want);
                 uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(fetch, nw);
-                base = __shfl(base, leader) + nthreads;
-                if (base + nw >= count) drained = true;
+                if ((int)lane == leader) base = atomicAdd(fetch, (uint32_t)__popcll(want));
+                base = __shfl(base, leader);
+                const uint32_t k = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(want >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)want, 0u));
+                const uint32_t last = base + (uint32_t)__popcll(want);
+                drained = nthreads + ((last >> 6) * groups + group) * 64u + (last & 63u) >= count;
                 if (!active) {
-                    const uint32_t idx = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(want >> 32),
-                                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)want, 0u));
+                    const uint32_t idx = nthreads + ((k >> 6) * groups + group) * 64u + (k & 63u);
                     if (idx < count) start(idx);
                 }
             }
@@ -240,74 +269,115 @@ __device__ __forceinline__ void persistent_trace(const DevScene& S, const IO& io
         }
         // ---- traverse until too many lanes have finished (or to the end once drained)
         do {
-            if (active) {
+            if (active && !fin && qn <= kPend - 4) {
                 if constexpr (kStats) ++nv;
                 const float4* np = S.nodes4 + (size_t)cur * 8;
                 const float4 lx = np[0], ly = np[1], lz = np[2], hx = np[3], hy = np[4], hz = np[5];
                 const uint4 rf = reinterpret_cast<const uint4*>(np)[6];
-                // all four slabs unconditionally (empty slots masked afterwards), then
-                // order the slots by sort key with a 5-comparator min/max network
-                float e0 = box_hit(r, lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, tmin, tclose);
-                float e1 = box_hit(r, lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, tmin, tclose);
-                float e2 = box_hit(r, lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, tmin, tclose);
-                float e3 = box_hit(r, lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, tmin, tclose);
-                e0 = rf.x == kMiss ? INFINITY : e0;
-                e1 = rf.y == kMiss ? INFINITY : e1;
-                e2 = rf.z == kMiss ? INFINITY : e2;
-                e3 = rf.w == kMiss ? INFINITY : e3;
-                uint32_t key[4] = {order_key(e0, 0), order_key(e1, 1), order_key(e2, 2), order_key(e3, 3)};
-                cx(key[0], key[1]);
-                cx(key[2], key[3]);
-                cx(key[0], key[2]);
-                cx(key[1], key[3]);
-                cx(key[1], key[2]);
-                uint32_t c[4];
-                float e[4];
+                const float e[4] = {box_hit(r, lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, tmin, tclose),
+                                    box_hit(r, lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, tmin, tclose),
+                                    box_hit(r, lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, tmin, tclose),
+                                    box_hit(r, lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, tmin, tclose)};
+                const uint32_t c[4] = {rf.x, rf.y, rf.z, rf.w};
+                // each hit child's rank by sort key among the hit children of its kind (leaf or
+                // internal): 6 compares, and the lane masks are combined in scalar registers
+                bool leaf[4], inner[4], lt[4][4];
+                uint32_t key[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t sl = key[q] & 3u;
-                    c[q] = sl == 0 ? rf.x : (sl == 1 ? rf.y : (sl == 2 ? rf.z : rf.w));
-                    e[q] = key[q] >= kKeyMiss ? INFINITY : (sl == 0 ? e0 : (sl == 1 ? e1 : (sl == 2 ? e2 : e3)));
+                for (int i = 0; i < 4; ++i) {
+                    const bool hit = e[i] != INFINITY && c[i] != kMiss;
+                    leaf[i] = hit && (c[i] & kLeafBit);
+                    inner[i] = hit && !(c[i] & kLeafBit);
+                    key[i] = IO::kPosTmin ? order_key_pos(e[i], i) : order_key(e[i], i);
                 }
-                bool done = false;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const bool test = e[k] != INFINITY && (c[k] & kLeafBit) && !done;
-                    if (test) {
-                        const uint32_t s = c[k] & ~kLeafBit;
-                        const float4* tp = S.tris + (size_t)s * 3;
-                        const float4 ta = tp[0], tb = tp[1], tc = tp[2];
-                        float tt, uu, vv;
-                        if constexpr (kStats) ++nt;
-                        if (tri_hit(r, ta, tb, tc, tmin, tclose, tt, uu, vv)) {
-                            tclose = tt;
-                            hprim = s;
-                            hu = uu;
-                            hv = vv;
-                            if (anyhit) done = true;
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = i + 1; k < 4; ++k) {
+                        const bool less = key[i] < key[k];
+                        const bool same = (leaf[i] && leaf[k]) || (inner[i] && inner[k]);
+                        lt[i][k] = same && less;
+                        lt[k][i] = same && !less;
+                    }
+                uint32_t rank[4], nleaf = 0, ninner = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    rank[i] = 0;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k != i) rank[i] += lt[k][i] ? 1u : 0u;
+                    nleaf += leaf[i] ? 1u : 0u;
+                    ninner += inner[i] ? 1u : 0u;
+                }
+                // leaves join the queue nearest first; a node's first one keeps the leaf bit
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (leaf[i])
+                        pend[((qh + qn + rank[i]) & (kPend - 1)) * kTraceBlock] =
+                            make_uint2(rank[i] == 0 ? c[i] : c[i] & ~kLeafBit, __float_as_uint(e[i]));
+                qn += nleaf;
+                // internal children go on the stack, the nearest on top, and the top is next
+                sp += ninner;
+                if (sp <= kStackLds) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (inner[i]) lds_col[(sp - 1 - rank[i]) * kTraceBlock] = c[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t at = sp - 1 - rank[i];
+                        if (inner[i]) {
+                            if (at < kStackLds) lds_col[at * kTraceBlock] = c[i];
+                            else ovf[at - kStackLds] = c[i];
                         }
                     }
                 }
-                if (!done) {
-                    // internal children still within the closest hit: nearest next, the rest pushed farthest first
-                    bool go[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) go[k] = e[k] != INFINITY && !(c[k] & kLeafBit) && e[k] <= tclose;
-                    const int f = go[0] ? 0 : (go[1] ? 1 : (go[2] ? 2 : (go[3] ? 3 : 4)));
-                    if (f == 4) {
-                        if (st.empty()) done = true;
-                        else cur = st.pop(lds_col, ovf);
-                    } else {
-#pragma unroll
-                        for (int k = 3; k >= 1; --k)
-                            if (go[k] && k > f) st.push(c[k], lds_col, ovf);
-                        cur = f == 0 ? c[0] : (f == 1 ? c[1] : (f == 2 ? c[2] : c[3]));
-                    }
+                if (sp == 0) {
+                    fin = true;
+                } else {
+                    --sp;
+                    cur = sp < kStackLds ? lds_col[sp * kTraceBlock] : ovf[sp - kStackLds];
                 }
-                if (done) {
+                if (fin && qn == 0) {
                     io.store(S, j, make_float4(tclose, __uint_as_float(hprim), hu, hv));
                     active = false;
                 }
+            }
+            // ---- intersect queued leaves once enough lanes have some, or no lane can step
+            uint32_t busy = (uint32_t)__popcll(__ballot(active));
+            uint32_t waiting = (uint32_t)__popcll(__ballot(active && qn > 0));
+            const bool stuck = __ballot(active && !fin && qn <= kPend - 4) == 0;
+            if (waiting > 0 && (stuck || waiting * 8 >= busy * kDrainAt)) {
+                do {
+                    if (active && qn > 0) {
+                        const uint2 w = pend[qh * kTraceBlock];
+                        qh = (qh + 1) & (kPend - 1);
+                        --qn;
+                        if (w.x & kLeafBit) tgroup = tclose;
+                        bool done = fin && qn == 0;
+                        if (__uint_as_float(w.y) <= tgroup) {
+                            const uint32_t s = w.x & ~kLeafBit;
+                            const float4* tp = S.tris + (size_t)s * 3;
+                            const float4 ta = tp[0], tb = tp[1], tc = tp[2];
+                            float tt, uu, vv;
+                            if constexpr (kStats) ++nt;
+                            if (tri_hit(r, ta, tb, tc, tmin, tclose, tt, uu, vv)) {
+                                tclose = tt;
+                                hprim = s;
+                                hu = uu;
+                                hv = vv;
+                                if (anyhit) done = true;
+                            }
+                        }
+                        if (done) {
+                            io.store(S, j, make_float4(tclose, __uint_as_float(hprim), hu, hv));
+                            active = false;
+                            qn = 0;
+                        }
+                    }
+                    busy = (uint32_t)__popcll(__ballot(active));
+                    waiting = (uint32_t)__popcll(__ballot(active && qn > 0));
+                } while (waiting > 0 && waiting * 8 >= busy * kDrainTo);
             }
         } while (__popcll(__ballot(active)) >= (drained ? 1 : kRefillThreshold));
     }
@@ -328,15 +398,17 @@ __global__ __launch_bounds__(kTraceBlock) void k_extend(DevScene S, ExtendIO io,
                                                         uint32_t* __restrict__ fetch, uint32_t* __restrict__ ovf,
                                                         unsigned long long* __restrict__ stats) {
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
+    __shared__ uint2 pend[kPend * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x;
-    persistent_trace<0, kStats>(S, io, *count, fetch, lds + threadIdx.x, ovf + (size_t)g * kStackOvf, stats);
+    persistent_trace<0, kStats>(S, io, *count, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf, stats);
 }
 
 __global__ __launch_bounds__(kTraceBlock) void k_connect(DevScene S, ConnectIO io, const uint32_t* __restrict__ count,
                                                          uint32_t* __restrict__ fetch, uint32_t* __restrict__ ovf) {
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
+    __shared__ uint2 pend[kPend * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x;
-    persistent_trace<1, false>(S, io, *count, fetch, lds + threadIdx.x, ovf + (size_t)g * kStackOvf, nullptr);
+    persistent_trace<1, false>(S, io, *count, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf, nullptr);
 }
 
 template <bool kStats>
@@ -347,9 +419,10 @@ __global__ __launch_bounds__(kTraceBlock) void k_extend_connect(DevScene S, Fuse
                                                                 uint32_t* __restrict__ ovf,
                                                                 unsigned long long* __restrict__ stats) {
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
+    __shared__ uint2 pend[kPend * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x;
     io.n_ext = *count_ext;
-    persistent_trace<2, kStats>(S, io, io.n_ext + *count_sh, fetch, lds + threadIdx.x, ovf + (size_t)g * kStackOvf,
+    persistent_trace<2, kStats>(S, io, io.n_ext + *count_sh, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf,
                                 stats);
 }
 
@@ -358,9 +431,10 @@ __global__ __launch_bounds__(kTraceBlock) void k_ref_trace(DevScene S, RefFusedI
                                                            const uint32_t* __restrict__ count_sh,
                                                            uint32_t* __restrict__ fetch, uint32_t* __restrict__ ovf) {
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
+    __shared__ uint2 pend[kPend * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x;
     io.n_ext = *count_ext;
-    persistent_trace<2, false>(S, io, io.n_ext + *count_sh, fetch, lds + threadIdx.x, ovf + (size_t)g * kStackOvf,
+    persistent_trace<2, false>(S, io, io.n_ext + *count_sh, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf,
                                nullptr);
 }
 
@@ -368,11 +442,12 @@ template <bool kAnyHit>
 __global__ __launch_bounds__(kTraceBlock) void k_rays(DevScene S, RaysIO io, uint32_t n, uint32_t* __restrict__ fetch,
                                                       uint32_t* __restrict__ ovf) {
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
+    __shared__ uint2 pend[kPend * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x;
-    persistent_trace<kAnyHit ? 1 : 0, false>(S, io, n, fetch, lds + threadIdx.x, ovf + (size_t)g * kStackOvf, nullptr);
+    persistent_trace<kAnyHit ? 1 : 0, false>(S, io, n, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf, nullptr);
 }
 
-__global__ void k_zero(uint32_t* p) { *p = 0u; }
+__global__ __launch_bounds__(256) void k_zero_fetch(uint32_t* p) { p[blockIdx.x * 256 + threadIdx.x] = 0u; }
 
 uint32_t g_grid = 0;
 
@@ -440,7 +515,7 @@ void launch_ref_trace(const DevScene& S, const uint32_t* queue, const uint32_t* 
 void launch_trace_rays(const DevScene& S, const float4* rays, float4* hits, uint32_t n, uint32_t* fetch,
                        uint32_t* ovf, hipStream_t s, uint32_t max_blocks) {
     if (n == 0) return;
-    k_zero<<<1, 1, 0, s>>>(fetch);
+    k_zero_fetch<<<kFetchWords / 256, 256, 0, s>>>(fetch);
     RaysIO io{rays, hits, nullptr};
     uint32_t grid = std::min(trace_grid_blocks(), (n + kTraceBlock - 1) / kTraceBlock);
     if (max_blocks) grid = std::min(grid, max_blocks);
@@ -450,7 +525,7 @@ void launch_trace_rays(const DevScene& S, const float4* rays, float4* hits, uint
 void launch_occluded_rays(const DevScene& S, const float4* rays, uint32_t* out, uint32_t n, uint32_t* fetch,
                           uint32_t* ovf, hipStream_t s) {
     if (n == 0) return;
-    k_zero<<<1, 1, 0, s>>>(fetch);
+    k_zero_fetch<<<kFetchWords / 256, 256, 0, s>>>(fetch);
     RaysIO io{rays, nullptr, out};
     const uint32_t grid = std::min(trace_grid_blocks(), (n + kTraceBlock - 1) / kTraceBlock);
     k_rays<true><<<grid, kTraceBlock, 0, s>>>(S, io, n, fetch, ovf);

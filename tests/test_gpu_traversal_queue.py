@@ -1,0 +1,79 @@
+"""The traversal's leaf queue, stack and ray dealing against the sequential oracle,
+bit for bit: triangles that all overlap (four leaf hits in one node, a stack deeper
+than its LDS part), origins on box planes, distances from below zero, and ray
+counts around the blocks, the resident threads and the 64 fetch groups."""
+import numpy as np
+import pytest
+
+from ohao_engine_amd import ohpt
+from ohao_engine_amd import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+
+def scene(pos):
+    return S.Scene(pos=np.ascontiguousarray(pos, np.float32), mat=np.zeros(len(pos), np.uint32),
+                   materials=S.cornell_box().materials[:1], camera=S.cornell_box().camera)
+
+
+def overlapping(n, seed):
+    """Triangles that each span most of the unit cube."""
+    return np.random.default_rng(seed).random((n, 9), dtype=np.float32)
+
+
+def rays_in(lo, hi, n, seed, tmin=0.0, tmax=np.inf):
+    rng = np.random.default_rng(seed)
+    r = np.empty((n, 8), np.float32)
+    r[:, 0:3] = rng.uniform(lo, hi, (n, 3))
+    d = rng.standard_normal((n, 3))
+    axis = rng.random(n) < 0.2                  # along an axis: slabs of zero extent in two of them
+    d[axis] = np.eye(3)[rng.integers(0, 3, axis.sum())] * rng.choice([-1.0, 1.0], (axis.sum(), 1))
+    r[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    r[:, 3] = tmin
+    r[:, 7] = tmax
+    return r
+
+
+def check(oracle, pos, rays):
+    sc = scene(pos)
+    ctx = ohpt.Context(32, 32)
+    ctx.load_scene(sc)
+    got = ctx.trace_rays(rays)
+    occ = ctx.occluded_rays(rays)
+    ctx.close()
+    o = oracle.OracleScene(sc)
+    want, visits, _ = o.trace(rays)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(occ, o.occluded(rays))
+    return visits
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 17, 300, 20000])
+def test_overlapping_triangles(oracle, n):
+    print(f"overlapping {n}", flush=True)
+    pos = overlapping(n, n)
+    visits = check(oracle, pos, rays_in(-0.5, 1.5, 3000, n))
+    if n == 20000:
+        assert visits.max() > 200
+
+
+@pytest.mark.parametrize("tmin,tmax", [(-2.0, 3.0), (0.25, 0.75), (0.0, 0.0), (-1.0, -0.1)])
+def test_distance_ranges(oracle, tmin, tmax):
+    print(f"range {tmin} {tmax}", flush=True)
+    check(oracle, overlapping(500, 9), rays_in(0.0, 1.0, 4000, 5, tmin, tmax))
+
+
+def test_origins_on_box_planes(oracle):
+    pos = np.round(overlapping(400, 3) * 8) / 8        # boxes on a grid, and the origins too
+    rays = rays_in(0.0, 1.0, 6000, 7)
+    rays[:, 0:3] = np.round(rays[:, 0:3] * 8) / 8
+    check(oracle, pos, rays)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 129, 327679, 327681, 327680 + 64 * 64 + 1, 700001])
+def test_ray_counts(oracle, n):
+    """A 256-CU grid holds 327,680 threads; further rays are dealt in 64 groups."""
+    print(f"count {n}", flush=True)
+    sc = S.displaced_sphere(6, 0.2, 1)
+    V, F = sc[0], sc[3]
+    check(oracle, V[F.reshape(-1)].reshape(-1, 9), rays_in(-1.2, 1.2, n, n))
