@@ -546,9 +546,8 @@ size_t lbvh_scratch_bytes(uint32_t n) { return layout(n).total; }
 
 namespace {
 // World-space corners (and normals) of one mesh's triangles from its
-// object-space vertices, in double as the host's scene upload computes them
-// (fp contraction is off in this file), so a refit sees the same floats a
-// fresh upload would.
+// object-space vertices, in double without contraction (off in this file) as
+// world_triangle computes the emitters' on the host; commits and refits share it.
 __global__ __launch_bounds__(256) void k_transform_mesh(const float* __restrict__ vpos, const float* __restrict__ vnrm,
                                                         const uint32_t* __restrict__ idx, uint32_t nt,
                                                         MeshTransform x, float* __restrict__ tpos,
@@ -588,7 +587,19 @@ __global__ __launch_bounds__(256) void k_transform_mesh(const float* __restrict_
             for (int q = 0; q < 3; ++q) tnrm[(size_t)t * 9 + k * 3 + q] = n[q];
     }
 }
+
+__global__ __launch_bounds__(256) void k_gather_uv(const float* __restrict__ vuv, const uint32_t* __restrict__ idx,
+                                                   uint32_t nc, float* __restrict__ tuv) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;   // corner
+    if (i >= nc) return;
+    const float2 v = vuv ? reinterpret_cast<const float2*>(vuv)[idx[i]] : make_float2(0.0f, 0.0f);
+    reinterpret_cast<float2*>(tuv)[i] = v;
+}
 }  // namespace
+
+void launch_gather_uv(const float* vuv, const uint32_t* idx, uint32_t nt, float* tuv, hipStream_t s) {
+    if (nt) k_gather_uv<<<(uint32_t)(((uint64_t)nt * 3 + 255) / 256), 256, 0, s>>>(vuv, idx, nt * 3, tuv);
+}
 
 void launch_transform_mesh(const float* vpos, const float* vnrm, const uint32_t* idx, uint32_t nt,
                            const MeshTransform& x, float* tpos, float* tnrm, hipStream_t s) {

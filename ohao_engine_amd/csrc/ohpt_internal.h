@@ -46,6 +46,8 @@ struct MeshTransform {
 // first triangle). tnrm null: no normals; vnrm null with tnrm: geometric normals.
 void launch_transform_mesh(const float* vpos, const float* vnrm, const uint32_t* idx, uint32_t nt,
                            const MeshTransform& x, float* tpos, float* tnrm, hipStream_t s);
+// Corner uvs of one mesh (nt*6 floats into tuv); vuv null: zeros.
+void launch_gather_uv(const float* vuv, const uint32_t* idx, uint32_t nt, float* tuv, hipStream_t s);
 // After lbvh_build or lbvh_refit with the same buffers (scratch still holding
 // depths and the 4-wide numbering): writes the n4 x 128 B 4-wide nodes.
 hipError_t bvh4_collapse(const LbvhBuffers& b, float4* nodes4, hipStream_t s);
