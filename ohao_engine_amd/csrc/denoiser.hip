@@ -23,10 +23,11 @@
 //                  input channels) and all nine taps; K = pixels, 32 per MFMA step,
 //                  split over the block's waves; per-block partial sums go to a buffer
 //                  that a fixed-order reduction sums (deterministic weight gradients).
-//   k_conv_dma<NC> k_conv3x3's tiling for the layers without an upsampled or
+//   k_conv_dma     k_conv3x3's tiling for the layers without an upsampled or
 //                  feature input, each chunk's halo and weights staged by
 //                  global->LDS loads into a second pair of LDS buffers while the
-//                  previous chunk's MFMAs run.
+//                  previous chunk's MFMAs run; k_conv_ring is its persistent form.
+//   k_conv_stream, k_conv_features: the full-resolution layers of inference.
 // The input gradient reuses these kernels with the weights flipped and transposed.
 #include <cmath>
 #include <cstring>
@@ -470,12 +471,133 @@ __global__ __launch_bounds__(32 * RW) void k_conv3x3(ConvArgs a) {
     }
 }
 
+// ------------------------------------------ shared parts of the persistent convolutions
+// Fragments are multiplied with the weights as the first operand, and row r of tile ni
+// is output channel 8 (r / 4) + 4 ni + r % 4: lane (g, r16), register i of tile ni then
+// is channel 8 g + 4 ni + i of pixel r16, so a lane stores eight channels of its pixel
+// as 16 bytes and a row needs no transpose through LDS.
+__device__ __forceinline__ int w_row(int ni, int r16) { return (r16 >> 2) * 8 + ni * 4 + (r16 & 3); }
+// 16-byte slot of vector v in the LDS row of output channel n: the rows that a fragment
+// read takes from one bank group (n % 4 alike) differ in n / 8
+__device__ __forceinline__ int w_slot(int n, int v) { return v ^ ((n >> 3) & 3); }
+
+// This lane's biases of the 32 output channels from n0.
+__device__ __forceinline__ void load_bias(const ConvArgs& a, int n0, int g, float bias[2][4]) {
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n = n0 + g * 8 + ni * 4 + i;
+            bias[ni][i] = (a.bias && n < a.nb) ? a.bias[n] : 0.0f;
+        }
+}
+
+// A 16x16 tile's image and tile coordinates, advanced tile by tile.
+struct Tile { int b, y, x; };
+__device__ __forceinline__ Tile tile_at(const ConvArgs& a, int t) {
+    const int tpi = a.tiles_x * a.tiles_y, b = t / tpi, r = t - b * tpi, y = r / a.tiles_x;
+    return Tile{b, y, r - y * a.tiles_x};
+}
+__device__ __forceinline__ void advance(const ConvArgs& a, Tile& t) {
+    if (++t.x == a.tiles_x) {
+        t.x = 0;
+        if (++t.y == a.tiles_y) { t.y = 0; ++t.b; }
+    }
+}
+
+__device__ __forceinline__ uint2 pack4(const float v[4]) {
+    return make_uint2((uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16, (uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16);
+}
+
+// Biased (and rectified) values of one pixel's channels n0 + 8 g + 4 ni + i, stored;
+// returned as bf16 for the pooling.
+__device__ __forceinline__ void store_row(const ConvArgs& a, int b, int y, int x, int n0, int g, const f32x4 acc[2],
+                                          const float bias[2][4], uint4& q) {
+    float v[2][4];
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[ni][i] = acc[ni][i] + bias[ni][i];
+            if (a.relu) v[ni][i] = fmaxf(v[ni][i], 0.0f);
+        }
+    const uint2 lo = pack4(v[0]), hi = pack4(v[1]);
+    q = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    if (y >= a.H || x >= a.W) return;
+    const size_t pix = (size_t)(b * a.H + y) * a.W + x;
+    const int n = n0 + g * 8;
+    if (a.outf) {
+        float4* o = reinterpret_cast<float4*>(&a.outf[pix * a.np + n]);
+        o[0] = make_float4(v[0][0], v[0][1], v[0][2], v[0][3]);
+        o[1] = make_float4(v[1][0], v[1][1], v[1][2], v[1][3]);
+    } else if (n < a.oc0) {
+        *reinterpret_cast<uint4*>(&a.out0[pix * a.oc0 + n]) = q;
+    } else {
+        *reinterpret_cast<uint4*>(&a.out1[pix * a.oc1 + (n - a.oc0)]) = q;
+    }
+}
+
+// 2x2 max-pool of two rows' stored values (top, bot: this lane's pixel), by the lanes
+// of even pixels; y, x: the pooled pixel. Origins, H and W are even.
+__device__ __forceinline__ void store_pooled(const ConvArgs& a, int b, int y, int x, int n0, int g, int r16,
+                                             const uint4& top, const uint4& bot) {
+    const int h2 = a.H >> 1, w2 = a.W >> 1;
+    auto other = [](const uint4& v) {
+        return make_uint4((uint32_t)__shfl_xor((int)v.x, 1), (uint32_t)__shfl_xor((int)v.y, 1),
+                          (uint32_t)__shfl_xor((int)v.z, 1), (uint32_t)__shfl_xor((int)v.w, 1));
+    };
+    const uint4 q[4] = {top, other(top), bot, other(bot)};
+    if ((r16 & 1) || y >= h2 || x >= w2) return;
+    *reinterpret_cast<uint4*>(&a.pool_out[((size_t)(b * h2 + y) * w2 + x) * a.np + n0 + g * 8]) = max4_bf16(q);
+}
+
+// One 32-channel input chunk for a wave's two output rows (from halo row row0) of 16
+// pixels x 32 output channels: a fragment of an input row serves both output rows that
+// it lies under, 12 + 18 LDS reads for 36 MFMAs. Per accumulator the taps run in
+// order (dy, then dx).
+__device__ __forceinline__ void conv_rows(const uint16_t* xs, const uint16_t* ws, int row0, int g, int r16,
+                                          f32x4 acc[2][2]) {
+    constexpr int HX = 18;
+    bf16x8 w[9][2];
+#pragma unroll
+    for (int ry = 0; ry < 4; ++ry) {
+        if (ry < 3) {
+#pragma unroll
+            for (int t = ry * 3; t < ry * 3 + 3; ++t)
+#pragma unroll
+                for (int ni = 0; ni < 2; ++ni)
+                    w[t][ni] = as_bf16x8(*reinterpret_cast<const uint4*>(
+                        &ws[(t * 32 + w_row(ni, r16)) * 32 + (w_slot(w_row(ni, r16), g) << 3)]));
+        }
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+            const int p = (row0 + ry) * HX + r16 + dx;
+            const bf16x8 x = as_bf16x8(*reinterpret_cast<const uint4*>(&xs[p * 32 + (halo_slot<32>(p, g) << 3)]));
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {
+                const int r = ry - dy;
+                if (r < 0 || r > 1) continue;
+#pragma unroll
+                for (int ni = 0; ni < 2; ++ni)
+                    acc[r][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dy * 3 + dx][ni], x, acc[r][ni], 0, 0, 0);
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ void zero_rows(f32x4 acc[2][2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
 // ------------------------------------- double-buffered convolution (LDS-direct loads)
 // Zero vector read by halo slots outside the image (an LDS-direct load cannot write
 // zeros of its own).
 __device__ __align__(16) uint32_t g_zero_vec[4] = {0u, 0u, 0u, 0u};
 
-// k_conv_dma<NC>: k_conv3x3<32, 1, 16, NC, false> with the staging of input chunk
+// k_conv_dma: k_conv3x3<32, 1, 16, 1, false> with the staging of input chunk
 // c + 1 (its 18x18 halo and packed weights) issued as global->LDS loads
 // (global_load_lds_dwordx4) into a second pair of LDS buffers before chunk c's
 // MFMAs, so the loads' latency hides behind the matrix work instead of
@@ -483,9 +605,8 @@ __device__ __align__(16) uint32_t g_zero_vec[4] = {0u, 0u, 0u, 0u};
 // 16-byte slot 64 i + l, so each lane fetches the vector that the XOR-swizzled
 // layouts of k_conv3x3 keep in that slot. The MFMA order per accumulator
 // (chunks, then K steps) and the epilogue are k_conv3x3's: bit-identical outputs.
-template <int NC>
 __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
-    constexpr int CC = 32, RW = 16, TX = 16, NT = 512, NO = 32 * NC, KS = 9;
+    constexpr int CC = 32, RW = 16, TX = 16, NT = 512, NO = 32, KS = 9;
     constexpr int HX = TX + 2, HP = HX * (RW + 2);   // 18 x 18 halo pixels
     constexpr int HSLOT = HP * 4;                    // 16-byte halo slots
     constexpr int WSLOT = KS * NO * 4;               // 16-byte weight slots
@@ -532,19 +653,19 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
         }
     };
 
-    f32x4 acc[2][2 * NC];
+    f32x4 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2 * NC; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto compute = [&](const uint16_t* xsb, const uint16_t* wsb) {
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             const int dy = s / 3, dx = s - dy * 3;   // 32-channel chunks: one tap per K step
-            bf16x8 bfr[2 * NC];
+            bf16x8 bfr[2];
 #pragma unroll
-            for (int ni = 0; ni < 2 * NC; ++ni)
+            for (int ni = 0; ni < 2; ++ni)
                 bfr[ni] = as_bf16x8(
                     *reinterpret_cast<const uint4*>(&wsb[(s * NO + ni * 16 + r16) * 32 + ((g ^ ((r16 >> 1) & 3)) << 3)]));
 #pragma unroll
@@ -552,7 +673,7 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
                 const int p = (wave * 2 + mi + dy) * HX + r16 + dx;
                 const bf16x8 af = as_bf16x8(*reinterpret_cast<const uint4*>(&xsb[p * CC + ((g ^ ((p >> 1) & 3)) << 3)]));
 #pragma unroll
-                for (int ni = 0; ni < 2 * NC; ++ni)
+                for (int ni = 0; ni < 2; ++ni)
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[ni], acc[mi][ni], 0, 0, 0);
             }
         }
@@ -586,7 +707,7 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
             const int y = y0 + wave * 2 + mi;
             if (y >= a.H) continue;
 #pragma unroll
-            for (int ni = 0; ni < 2 * NC; ++ni) {
+            for (int ni = 0; ni < 2; ++ni) {
                 const int n = nc * NO + ni * 16 + r16;
                 const float bias = (a.bias && n < a.nb) ? a.bias[n] : 0.0f;
 #pragma unroll
@@ -604,13 +725,13 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
     }
     // bf16 outputs: the tile transposed through LDS ([pixel][NO channels], padded)
     constexpr int OS = NO + 8;
-    static_assert(RW * TX * OS <= (NC == 1 ? HP * CC : KS * NO * 32), "output staging fits its buffer");
-    uint16_t* os = NC == 1 ? xa : wa;
+    static_assert(RW * TX * OS <= HP * CC, "output staging fits its buffer");
+    uint16_t* os = xa;
     __syncthreads();
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi) {
 #pragma unroll
-        for (int ni = 0; ni < 2 * NC; ++ni) {
+        for (int ni = 0; ni < 2; ++ni) {
             const int nl = ni * 16 + r16, n = nc * NO + nl;
             const float bias = (a.bias && n < a.nb) ? a.bias[n] : 0.0f;
 #pragma unroll
@@ -622,8 +743,8 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
         }
     }
     __syncthreads();
-    for (int i = tid; i < RW * TX * 4 * NC; i += NT) {
-        const int pl = i / (4 * NC), v = i % (4 * NC);
+    for (int i = tid; i < RW * TX * 4; i += NT) {
+        const int pl = i / (4), v = i % (4);
         const int y = y0 + pl / TX, x = x0 + pl % TX;
         if (y >= a.H || x >= a.W) continue;
         const uint4 val = *reinterpret_cast<const uint4*>(&os[pl * OS + v * 8]);
@@ -634,8 +755,8 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
     }
     if (a.pool_out) {
         const int h2 = a.H >> 1, w2 = a.W >> 1;
-        for (int i = tid; i < (RW / 2) * (TX / 2) * 4 * NC; i += NT) {
-            const int pl = i / (4 * NC), v = i % (4 * NC);
+        for (int i = tid; i < (RW / 2) * (TX / 2) * 4; i += NT) {
+            const int pl = i / (4), v = i % (4);
             const int py = pl / (TX / 2), px = pl % (TX / 2);
             const int y = (y0 >> 1) + py, x = (x0 >> 1) + px;
             if (y >= h2 || x >= w2) continue;
@@ -649,6 +770,130 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
     }
 }
 
+// k_conv_ring: k_conv_dma's tile and staging, persistent: a block keeps its 32 output
+// channels and walks a range of tiles, and the (tile, chunk) steps take the two pairs of
+// LDS buffers in turn across tile borders, so a layer of one chunk overlaps its loads
+// too and a tile's stores drain behind the next step's MFMAs. With one or two chunks
+// the weights stay in LDS; halo addresses are kept per lane, border checks only where
+// a tile has a border. Bounded by the latency of the halo loads (two blocks per CU,
+// 78 KB each) and the LDS reads. 1920x1080 with / without: 32 -> 64 channels at half
+// size 34 / 43 us, 64 -> 64 52 / 64 us (740 TFLOP/s), 96 -> 96 at a quarter 35 / 36 us.
+// Below two tiles and channel groups per resident block its longer prologue costs
+// 0.5-1 us a layer, and k_conv_dma runs.
+__global__ __launch_bounds__(512, 4) void k_conv_ring(ConvArgs a) {
+    constexpr int CC = 32, RW = 16, TX = 16, NO = 32, KS = 9;
+    constexpr int HX = TX + 2, HP = HX * (RW + 2);   // 18 x 18 halo pixels
+    constexpr int HSLOT = HP * 4;                    // 16-byte halo slots
+    constexpr int WSLOT = KS * NO * 4;               // 16-byte weight slots
+    constexpr int HI = (HSLOT + 63) / 64, WI = WSLOT / 64;
+    constexpr int NW = 8;
+    __shared__ __align__(16) uint16_t xa[HP * CC];
+    __shared__ __align__(16) uint16_t xb[HP * CC];
+    __shared__ __align__(16) uint16_t wa[KS * NO * 32];
+    __shared__ __align__(16) uint16_t wb[KS * NO * 32];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, r16 = lane & 15;
+    const int ncout = a.np / NO;
+    const int nchunk = (a.c0 + a.c1) / CC;
+    // XCD-banded order (workgroups are dealt round-robin to the 8 XCDs): the blocks of a
+    // tile range, one per 32 output channels, run on one XCD and share its L2
+    int lb = blockIdx.x;
+    if ((gridDim.x & 7) == 0) lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int range = lb / ncout, nc = lb - range * ncout;
+    const int t_begin = range * a.per_block, t_end = min(t_begin + a.per_block, a.B * a.tiles_x * a.tiles_y);
+    if (t_begin >= t_end) return;   // whole block: before any barrier
+    const int nsteps = (t_end - t_begin) * nchunk;
+    Tile nt = tile_at(a, t_begin);   // tile of the next step to stage
+
+    // where this lane's slots of a halo and of a chunk's weights lie: the same for every tile
+    constexpr int HK = (HI + NW - 1) / NW, WK = (WI + NW - 1) / NW;
+    int hpix[HK], hyx[HK], woff[WK];   // pixel offset from the halo's corner * 4 + vector; hy << 8 | hx
+#pragma unroll
+    for (int k = 0; k < HK; ++k) {
+        const int s = (wave + k * NW) * 64 + lane, p = s >> 2, v = (s & 3) ^ ((p >> 1) & 3);
+        const int hy = p / HX, hx = p - hy * HX;
+        hpix[k] = (hy * a.W + hx) * 4 + v;
+        hyx[k] = hy << 8 | hx;
+    }
+#pragma unroll
+    for (int k = 0; k < WK; ++k) {
+        const int s = (wave + k * NW) * 64 + lane, row = s >> 2, st = row / NO, n = row - st * NO;
+        woff[k] = (st * a.np + n) * 32 + w_slot(n, s & 3) * 8;
+    }
+    Tile ct = nt;           // tile of the computed step
+    int nch = 0, cch = 0;   // their chunks
+    auto issue = [&](bool weights, uint16_t* xd, uint16_t* wd) __attribute__((always_inline)) {
+        const int cb = nch * CC;
+        const uint16_t* src;
+        int cs, co;
+        if (cb < a.c0) { src = a.in0; cs = a.c0; co = cb; }
+        else { src = a.in1; cs = a.c1; co = cb - a.c0; }
+        const int x0 = nt.x * TX - 1, y0 = nt.y * RW - 1;   // the halo's corner
+        const uint16_t* img = src + ((int64_t)nt.b * a.H * a.W + (int64_t)y0 * a.W + x0) * cs + co;
+        const bool inside = x0 >= 0 && y0 >= 0 && x0 + HX <= a.W && y0 + RW + 2 <= a.H;
+#pragma unroll
+        for (int k = 0; k < HK; ++k) {
+            const int i = wave + k * NW;
+            if (i * 64 + lane >= HSLOT) continue;
+            const void* gp = img + ((uint32_t)(hpix[k] >> 2) * (uint32_t)cs + (hpix[k] & 3) * 8);
+            if (!inside) {
+                const int gy = y0 + (hyx[k] >> 8), gx = x0 + (hyx[k] & 255);
+                if (gy < 0 || gy >= a.H || gx < 0 || gx >= a.W) gp = g_zero_vec;
+            }
+            __builtin_amdgcn_global_load_lds(gp, xd + i * 64 * 8, 16, 0, 0);
+        }
+        if (weights) {
+            const uint16_t* wsrc = a.wp + ((size_t)nch * KS * a.np + (size_t)nc * NO) * 32;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) {
+                const int i = wave + k * NW;
+                if (i >= WI) continue;
+                const void* wp = wsrc + woff[k];
+                __builtin_amdgcn_global_load_lds(wp, wd + i * 64 * 8, 16, 0, 0);
+            }
+        }
+        if (++nch == nchunk) { nch = 0; advance(a, nt); }
+    };
+    // This wave's LDS-direct loads have landed before it reaches a barrier, so after
+    // the barrier the whole buffer is written.
+    auto loads_then_barrier = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+
+    float bias[2][4];
+    f32x4 acc[2][2];
+    zero_rows(acc);
+    auto step = [&](int j, const uint16_t* xs, const uint16_t* ws, uint16_t* xn, uint16_t* wn)
+                    __attribute__((always_inline)) {
+        // with one or two chunks each buffer keeps its chunk's weights
+        if (j + 1 < nsteps) issue(j == 0 || nchunk > 2, xn, wn);
+        conv_rows(xs, ws, wave * 2, g, r16, acc);
+        loads_then_barrier();   // step j + 1 staged; (xs, ws) no longer read
+        if (++cch == nchunk) {   // the stores drain behind the next step's MFMAs
+            const int y = ct.y * RW + wave * 2, x = ct.x * TX + r16;
+            uint4 q[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) store_row(a, ct.b, y + r, x, nc * NO, g, acc[r], bias, q[r]);
+            if (a.pool_out) store_pooled(a, ct.b, y >> 1, x >> 1, nc * NO, g, r16, q[0], q[1]);
+            zero_rows(acc);
+            cch = 0;
+            advance(a, ct);
+        }
+    };
+
+    issue(true, xa, wa);
+    load_bias(a, nc * NO, g, bias);
+    loads_then_barrier();
+    int j = 0;
+    for (; j + 1 < nsteps; j += 2) {
+        step(j, xa, wa, xb, wb);
+        step(j + 1, xb, wb, xa, wa);
+    }
+    if (j < nsteps) step(j, xa, wa, xb, wb);
+}
+
 // ------------------------------------------- streaming full-resolution convolution
 // LDS writes of this wave are visible to its other lanes after this (no block barrier).
 __device__ inline void wave_lds_sync() {
@@ -657,39 +902,34 @@ __device__ inline void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// k_conv_stream<CC, NCH, EPI>: inference convolutions with 32 output
-// channels on the full-resolution 16-aligned grid, NCH input chunks of CC
-// channels. Persistent: a block (8 waves, 512 threads) stages the layer's
-// packed weights in LDS once and walks a contiguous range of 16x16 output
-// tiles. Each (tile, chunk) step stages its 18x18 halo in one of two LDS
-// buffers; the global loads of the next step are issued before this step's
-// MFMAs and converted (bilinear upsample, guide features) after them, so HBM
-// latency hides behind the matrix work with one block barrier per step. Each
-// wave owns two output rows and finishes its tile in a private LDS stage
-// (bf16 transpose to 16-byte stores, 2x2 max-pool, or the kernel-prediction
-// filter) without a block barrier. Halo pixels and weight rows are stored
-// unpadded with their 16-byte vectors XOR-swizzled by the pixel (row) index,
-// so a 16-lane fragment read spreads over the banks and two blocks fit per CU.
-// The per-accumulator MFMA order (chunks, then K steps) is k_conv3x3's, so
-// the convolution outputs are bit-identical to it.
-//   CC = 16: the input is the 16 guide features (a.feat); EPI 0: bf16 store,
-//   1: + 2x2 max-pool, 2: the head (25 logits) with the kernel prediction
-//   applied to a.kpn_rad (the tile's 20x20 radiance window is staged in LDS;
-//   four lanes per pixel share the 25 taps).
+// k_conv_stream<EPI>: inference convolutions 32 -> 32 channels on the full-resolution
+// 16-aligned grid. Persistent: a block (8 waves, 512 threads) stages the layer's
+// packed weights in LDS once and walks a contiguous range of 16x16 output tiles. Each
+// tile's 18x18 halo goes to one of two LDS buffers; the global loads of the next tile
+// are issued before this tile's MFMAs, so HBM latency hides behind the matrix work
+// with one block barrier per tile. Each wave owns two output rows and finishes its
+// tile in a private LDS stage (bf16 transpose to 16-byte stores, 2x2 max-pool, or the
+// kernel-prediction filter) without a block barrier. Halo pixels and weight rows are
+// stored unpadded with their 16-byte vectors XOR-swizzled by the pixel (row) index, so
+// a 16-lane fragment read spreads over the banks and two blocks fit per CU. The
+// per-accumulator MFMA order is k_conv3x3's, so the outputs are bit-identical to it.
+//   EPI 0: bf16 store, 1: + 2x2 max-pool, 2: the head (25 logits) with the kernel
+//   prediction applied to a.kpn_rad (the tile's 20x20 radiance window is staged in
+//   LDS; four lanes per pixel share the 25 taps).
 // The decoder's upsampling layers stay on k_conv3x3 (measured faster there:
 // the interpolation registers and three chunks of weights leave one block per CU).
 constexpr int kStreamNT = 512;
 
-template <int CC, int NCH, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
-    constexpr int NT = kStreamNT, TX = 16, RW = 16, HX = TX + 2, HP = HX * (RW + 2);
-    constexpr int KS = (9 * CC + 31) / 32;
+    constexpr int CC = 32, NT = kStreamNT, TX = 16, RW = 16, HX = TX + 2, HP = HX * (RW + 2);
+    constexpr int KS = 9;
     constexpr int VPP = CC / 8;
     constexpr int PSTEP = NT / VPP, NPF = (HP + PSTEP - 1) / PSTEP;
     constexpr int XB = HP * CC;                                      // halo buffer (bf16 units)
     constexpr int OS = 40;                                           // staged pixel stride (bf16)
     constexpr int OSW = EPI == 2 ? TX * 25 * 2 : 2 * TX * OS;        // per-wave stage (bf16 units)
-    constexpr int WL = NCH * KS * 32 * 32;
+    constexpr int WL = KS * 32 * 32;
     __shared__ __align__(16) uint16_t xs[2 * XB];
     __shared__ __align__(16) uint16_t os[(NT / 64) * OSW];
     __shared__ __align__(16) uint16_t ws[WL];
@@ -707,11 +947,11 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
     const int tpi = a.tiles_x * a.tiles_y;
     const int t_begin = lb * a.per_block, t_end = min(t_begin + a.per_block, a.B * tpi);
     if (t_begin >= t_end) return;   // whole block: before any barrier
-    const int nsteps = (t_end - t_begin) * NCH;
+    const int nsteps = t_end - t_begin;
 
-    // packed weights [chunk][step][n][32] -> LDS rows of 32 bf16, vectors swizzled by the row
-    for (int i = tid; i < NCH * KS * 32 * 4; i += NT) {
-        const int sn = i >> 2, v = i & 3;   // sn = (chunk * KS + step) * 32 + output channel
+    // packed weights [step][n][32] -> LDS rows of 32 bf16, vectors swizzled by the row
+    for (int i = tid; i < KS * 32 * 4; i += NT) {
+        const int sn = i >> 2, v = i & 3;   // sn = step * 32 + output channel
         *reinterpret_cast<uint4*>(&ws[sn * 32 + ((v ^ ((sn >> 1) & 3)) << 3)]) =
             *reinterpret_cast<const uint4*>(a.wp + ((size_t)(sn >> 5) * a.np + (sn & 31)) * 32 + v * 8);
     }
@@ -725,7 +965,6 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
     // halo slots of this thread: pixel tid / VPP + k * PSTEP, 16-byte vector tid % VPP
     const int hv = tid % VPP;
     uint4 pv[NPF];
-    Feat8 pf[CC == 16 ? NPF : 1];
     uint32_t inb = 0;      // bit k: slot k inside the image
     float4 pr = make_float4(0.f, 0.f, 0.f, 0.f);   // head: this thread's radiance window texel
 
@@ -738,13 +977,8 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
     // issue the global loads of step j
     auto issue = [&](int j) {
         int b, x0, y0;
-        tile_origin(t_begin + j / NCH, b, x0, y0);
-        const int cb = (j % NCH) * CC;
-        const uint16_t* src;
-        int cs, co;
-        if (cb < a.c0) { src = a.in0; cs = a.c0; co = cb; }
-        else { src = a.in1; cs = a.c1; co = cb - a.c0; }
-        const uint16_t* img = src + (size_t)b * a.H * a.W * cs + co + hv * 8;
+        tile_origin(t_begin + j, b, x0, y0);
+        const uint16_t* img = a.in0 + (size_t)b * a.H * a.W * CC + hv * 8;
         inb = 0;
 #pragma unroll
         for (int k = 0; k < NPF; ++k) {
@@ -753,11 +987,7 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
             const int gy = y0 - 1 + hy, gx = x0 - 1 + hx;
             const bool in = p < HP && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W;
             inb |= (uint32_t)in << k;
-            if constexpr (CC == 16) {
-                if (in) pf[k] = feat_load(a.feat, b, gy, gx, hv);
-            } else {
-                if (in) pv[k] = *reinterpret_cast<const uint4*>(img + ((size_t)gy * a.W + gx) * cs);
-            }
+            if (in) pv[k] = *reinterpret_cast<const uint4*>(img + ((size_t)gy * a.W + gx) * CC);
         }
         if constexpr (EPI == 2) {
             if (tid < RWN) {
@@ -767,21 +997,16 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
             }
         }
     };
-    // convert the loaded values of the pending step into halo vectors (guide features)
     auto finish = [&]() {
 #pragma unroll
-        for (int k = 0; k < NPF; ++k) {
-            const bool in = (inb >> k) & 1u;
-            if constexpr (CC == 16) pv[k] = in ? feat_mix(a.feat, pf[k], hv) : make_uint4(0u, 0u, 0u, 0u);
-            else if (!in) pv[k] = make_uint4(0u, 0u, 0u, 0u);
-        }
+        for (int k = 0; k < NPF; ++k)
+            if (!((inb >> k) & 1u)) pv[k] = make_uint4(0u, 0u, 0u, 0u);
     };
 
     issue(0);
     finish();
     f32x4 acc[2][2];
     for (int j = 0; j < nsteps; ++j) {
-        const int c = j % NCH;
         uint16_t* xb = xs + (j & 1) * XB;
 #pragma unroll
         for (int k = 0; k < NPF; ++k) {
@@ -791,39 +1016,30 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
         __syncthreads();   // halo j (and, at j = 0, the weights) complete; step j - 1's buffer is free
         if constexpr (EPI == 2) {
             // every wave has finished step j - 1's filter: the window of tile j replaces it
-            if (c == 0 && tid < RWN) rwin[tid] = pr;
+            if (tid < RWN) rwin[tid] = pr;
         }
         if (j + 1 < nsteps) issue(j + 1);
-        if (c == 0) {
-#pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-                for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        zero_rows(acc);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            const int kf = s * 32 + g * 8;
-            const int tap = kf / CC, ci0 = kf - tap * CC;
-            const int dy = tap / 3, dx = tap - dy * 3;
+            const int dy = s / 3, dx = s - dy * 3;
             bf16x8 bfr[2];
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni)
                 bfr[ni] = as_bf16x8(*reinterpret_cast<const uint4*>(
-                    &ws[((c * KS + s) * 32 + ni * 16 + r16) * 32 + ((g ^ ((r16 >> 1) & 3)) << 3)]));
+                    &ws[(s * 32 + ni * 16 + r16) * 32 + ((g ^ ((r16 >> 1) & 3)) << 3)]));
 #pragma unroll
             for (int mi = 0; mi < 2; ++mi) {
                 const int p = (wave * 2 + mi + dy) * HX + r16 + dx;
-                uint4 v = make_uint4(0u, 0u, 0u, 0u);
-                if (tap < 9) v = *reinterpret_cast<const uint4*>(&xb[p * CC + (halo_slot<CC>(p, ci0 >> 3) << 3)]);
-                const bf16x8 af = as_bf16x8(v);
+                const bf16x8 af = as_bf16x8(*reinterpret_cast<const uint4*>(&xb[p * CC + (halo_slot<CC>(p, g) << 3)]));
 #pragma unroll
                 for (int ni = 0; ni < 2; ++ni)
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[ni], acc[mi][ni], 0, 0, 0);
             }
         }
-        if (c == NCH - 1) {
+        {
             int b, x0, y0;
-            tile_origin(t_begin + j / NCH, b, x0, y0);
+            tile_origin(t_begin + j, b, x0, y0);
             uint16_t* st = os + wave * OSW;
             if constexpr (EPI == 2) {
                 // one row at a time: its 16 pixels' 25 logits through this wave's LDS stage,
@@ -929,6 +1145,96 @@ __global__ __launch_bounds__(kStreamNT) void k_conv_stream(ConvArgs a) {
             }
         }
         if (j + 1 < nsteps) finish();
+    }
+}
+
+// The input layer of inference: k_conv_stream's persistent form over the 16 guide
+// features. A thread loads the guides of one halo pixel and converts all of them (a
+// thread per half pixel made every wave run both halves, twice), the fragments are
+// multiplied as in conv_rows. 1920x1080: 118 -> 97 us; HBM 45 us (273 MB).
+__global__ __launch_bounds__(kStreamNT, 4) void k_conv_features(ConvArgs a) {
+    constexpr int CC = 16, NT = kStreamNT, HX = 18, HP = HX * 18, KS = 5;
+    __shared__ __align__(16) uint16_t xs[2 * HP * CC];
+    __shared__ __align__(16) uint16_t ws[KS * 32 * 32];
+    static_assert(NT >= HP, "a halo pixel per thread");
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int g = lane >> 4, r16 = lane & 15;
+    int lb = blockIdx.x;   // XCD-banded order, as k_conv_stream
+    if ((gridDim.x & 7) == 0) lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int t_begin = lb * a.per_block, t_end = min(t_begin + a.per_block, a.B * a.tiles_x * a.tiles_y);
+    if (t_begin >= t_end) return;   // whole block: before any barrier
+    const int nsteps = t_end - t_begin;
+
+    for (int i = tid; i < KS * 32 * 4; i += NT) {
+        const int sn = i >> 2, v = i & 3;   // sn = step * 32 + output channel
+        *reinterpret_cast<uint4*>(&ws[sn * 32 + (w_slot(sn & 31, v) << 3)]) =
+            *reinterpret_cast<const uint4*>(a.wp + ((size_t)(sn >> 5) * a.np + (sn & 31)) * 32 + v * 8);
+    }
+    float bias[2][4];
+    load_bias(a, 0, g, bias);
+
+    const int hy = tid / HX, hx = tid - hy * HX;   // this thread's halo pixel
+    float4 fr, fa, fn;                             // its guides
+    float fd = 0.0f;
+    bool in = false;                               // inside the image
+    Tile nt = tile_at(a, t_begin), ct = nt;        // the next tile to load, the computed one
+    auto issue = [&]() {
+        const int gy = nt.y * 16 - 1 + hy, gx = nt.x * 16 - 1 + hx;
+        in = tid < HP && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W;
+        if (in) {
+            const size_t q = ((size_t)nt.b * a.feat.H + min(gy, a.feat.H - 1)) * a.feat.W + min(gx, a.feat.W - 1);
+            fr = a.feat.rad[q];
+            fa = a.feat.alb ? a.feat.alb[q] : make_float4(0, 0, 0, 0);
+            fn = a.feat.nrm ? a.feat.nrm[q] : make_float4(0, 0, 0, 0);
+            fd = a.feat.dep ? a.feat.dep[q] : 0.0f;
+        }
+        advance(a, nt);
+    };
+    auto stage = [&](int buf) {
+        if (tid >= HP) return;
+        uint16_t* xb = xs + buf * HP * CC;
+        uint4 lo = make_uint4(0u, 0u, 0u, 0u), hi = lo;
+        if (in) {
+            lo = feat_mix(a.feat, Feat8{fr, fa, fn}, 0);
+            hi = feat_mix(a.feat, Feat8{make_float4(fd, 0, 0, 0), fa, fn}, 1);
+        }
+        *reinterpret_cast<uint4*>(&xb[tid * CC + (halo_slot<CC>(tid, 0) << 3)]) = lo;
+        *reinterpret_cast<uint4*>(&xb[tid * CC + (halo_slot<CC>(tid, 1) << 3)]) = hi;
+    };
+
+    issue();
+    stage(0);
+    for (int j = 0; j < nsteps; ++j) {
+        const uint16_t* xb = xs + (j & 1) * HP * CC;
+        __syncthreads();   // tile j staged; the other buffer is no longer read
+        if (j + 1 < nsteps) issue();
+        f32x4 acc[2][2];
+        zero_rows(acc);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            bf16x8 w[2];
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+                w[ni] = as_bf16x8(*reinterpret_cast<const uint4*>(
+                    &ws[(s * 32 + w_row(ni, r16)) * 32 + (w_slot(w_row(ni, r16), g) << 3)]));
+            const int tap = s * 2 + (g >> 1), dy = tap / 3, dx = tap - dy * 3;   // two taps per K step
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int p = (wave * 2 + r + dy) * HX + r16 + dx;
+                uint4 v = make_uint4(0u, 0u, 0u, 0u);
+                if (tap < 9) v = *reinterpret_cast<const uint4*>(&xb[p * CC + (halo_slot<CC>(p, g & 1) << 3)]);
+#pragma unroll
+                for (int ni = 0; ni < 2; ++ni)
+                    acc[r][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[ni], as_bf16x8(v), acc[r][ni], 0, 0, 0);
+            }
+        }
+        uint4 q;
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            store_row(a, ct.b, ct.y * 16 + wave * 2 + r, ct.x * 16 + r16, 0, g, acc[r], bias, q);
+        advance(a, ct);
+        if (j + 1 < nsteps) stage((j + 1) & 1);
     }
 }
 
@@ -1576,19 +1882,16 @@ constexpr int kConvRows = 16;
 // Persistent streaming launch over the 16x16 tiles: as many blocks per compute
 // unit as its registers and LDS allow (measured once per kernel), rounded up to
 // a multiple of the 8 XCDs.
-template <int CC, int NCH, int EPI>
-void launch_stream(ohpt_denoiser* d, ConvArgs a) {
-    static int per_cu = 0;
+template <class K>
+void launch_stream(ohpt_denoiser* d, ConvArgs a, K kernel, int& per_cu) {
     if (per_cu <= 0 &&
-        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_conv_stream<CC, NCH, EPI>, kStreamNT, 0) !=
-             hipSuccess ||
-         per_cu <= 0))
+        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kStreamNT, 0) != hipSuccess || per_cu <= 0))
         per_cu = 1;
     const int n_tiles = a.B * a.tiles_x * a.tiles_y;
     const int max_blocks = std::max(8, per_cu * d->num_cus);
     a.per_block = (int)cdiv(n_tiles, max_blocks);
     const int nb = ((int)cdiv(n_tiles, a.per_block) + 7) & ~7;
-    k_conv_stream<CC, NCH, EPI><<<nb, kStreamNT, 0, d->stream>>>(a);
+    kernel<<<nb, kStreamNT, 0, d->stream>>>(a);
 }
 
 void launch_conv(ohpt_denoiser* d, const Layer& L, const ConvArgs& a, int cc) {
@@ -1614,16 +1917,29 @@ void launch_conv(ohpt_denoiser* d, const Layer& L, const ConvArgs& a, int cc) {
         (void)hipEventRecord(e0, d->stream);
     }
     if (a.tiles_x > 0) {
-        if (cc == 16) launch_stream<16, 1, 0>(d, a);
-        else if (a.kpn_out) launch_stream<32, 1, 2>(d, a);
-        else if (a.pool_out) launch_stream<32, 1, 1>(d, a);
-        else launch_stream<32, 1, 0>(d, a);
+        static int per_cu[4] = {};
+        if (cc == 16) launch_stream(d, a, k_conv_features, per_cu[3]);
+        else if (a.kpn_out) launch_stream(d, a, k_conv_stream<2>, per_cu[2]);
+        else if (a.pool_out) launch_stream(d, a, k_conv_stream<1>, per_cu[1]);
+        else launch_stream(d, a, k_conv_stream<0>, per_cu[0]);
     } else if (cc == 16) k_conv3x3<16, kConvMX, 8, 1, false><<<grid, 256, 0, d->stream>>>(a);
     else if (!a.up0) {
-        // 32 output channels per block: two blocks per CU (78 KB of LDS each);
-        // 64 per block (115 KB, one per CU) measured 3.5 % slower per inference
-        grid.z = (uint32_t)(a.B * (a.np / 32));
-        k_conv_dma<1><<<grid, 512, 0, d->stream>>>(a);
+        // 32 output channels per block: two blocks per CU (78 KB of LDS each); more than two
+        // tiles for each: the persistent form, a tile per block again until each would get
+        // three (fewer, longer blocks leave too many idle at the end). 540 tiles and groups
+        // on 512 resident blocks: 16.9 us without, 17.6 us with it; 1530: 26.2 and 25.8 us.
+        ConvArgs p = a;
+        p.tiles_x = (int)cdiv(a.W, 16);
+        p.tiles_y = (int)cdiv(a.H, 16);
+        const int ncout = a.np / 32, n_tiles = a.B * p.tiles_x * p.tiles_y;
+        const int64_t slots = 2ll * d->num_cus, work = (int64_t)n_tiles * ncout;
+        if (work <= 2 * slots) {
+            grid.z = (uint32_t)(a.B * ncout);
+            k_conv_dma<<<grid, 512, 0, d->stream>>>(a);
+        } else {
+            p.per_block = work < 3 * slots - ncout ? 1 : (int)cdiv(n_tiles, (uint64_t)std::max<int64_t>(1, slots / ncout));
+            k_conv_ring<<<(cdiv(n_tiles, p.per_block) * ncout + 7u) & ~7u, 512, 0, d->stream>>>(p);
+        }
     }
     else if (no == 64 && a.up0) k_conv3x3<32, kConvMX, kConvRows, 2, true><<<grid, 32 * kConvRows, 0, d->stream>>>(a);
     else k_conv3x3<32, kConvMX, kConvRows, 1, true><<<grid, 32 * kConvRows, 0, d->stream>>>(a);
