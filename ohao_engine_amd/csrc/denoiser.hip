@@ -217,6 +217,8 @@ struct ConvArgs {
     int oc0, oc1;
     float* outf;           // FP32 output with np channels (replaces out0/out1)
     int relu;
+    // input gradient: out0 is zeroed where this tensor (its layout) is not positive, or null
+    const uint16_t* mask0;
     int B, H, W;
     // in0 is the (H/2) x (W/2) image whose x2 bilinear upsample is the input
     // (the upsample is computed in the halo load instead of being stored)
@@ -509,6 +511,18 @@ __device__ __forceinline__ uint2 pack4(const float v[4]) {
     return make_uint2((uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16, (uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16);
 }
 
+// The gradients g of eight channels whose activations y are positive, the others 0. The
+// kernel that writes a gradient last masks it: a pass over each tensor took 238 us of a
+// 16 x 256^2 training step of 2.75 ms.
+__device__ __forceinline__ uint4 relu_masked(uint4 g, uint4 y) {
+    uint16_t* ge = reinterpret_cast<uint16_t*>(&g);
+    const uint16_t* ye = reinterpret_cast<const uint16_t*>(&y);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (!(bf2f(ye[k]) > 0.0f)) ge[k] = 0;
+    return g;
+}
+
 // Biased (and rectified) values of one pixel's channels n0 + 8 g + 4 ni + i, stored;
 // returned as bf16 for the pooling.
 __device__ __forceinline__ void store_row(const ConvArgs& a, int b, int y, int x, int n0, int g, const f32x4 acc[2],
@@ -531,7 +545,9 @@ __device__ __forceinline__ void store_row(const ConvArgs& a, int b, int y, int x
         o[0] = make_float4(v[0][0], v[0][1], v[0][2], v[0][3]);
         o[1] = make_float4(v[1][0], v[1][1], v[1][2], v[1][3]);
     } else if (n < a.oc0) {
-        *reinterpret_cast<uint4*>(&a.out0[pix * a.oc0 + n]) = q;
+        uint4 o = q;
+        if (a.mask0) o = relu_masked(q, *reinterpret_cast<const uint4*>(&a.mask0[pix * a.oc0 + n]));
+        *reinterpret_cast<uint4*>(&a.out0[pix * a.oc0 + n]) = o;
     } else {
         *reinterpret_cast<uint4*>(&a.out1[pix * a.oc1 + (n - a.oc0)]) = q;
     }
@@ -747,9 +763,10 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
         const int pl = i / (4), v = i % (4);
         const int y = y0 + pl / TX, x = x0 + pl % TX;
         if (y >= a.H || x >= a.W) continue;
-        const uint4 val = *reinterpret_cast<const uint4*>(&os[pl * OS + v * 8]);
+        uint4 val = *reinterpret_cast<const uint4*>(&os[pl * OS + v * 8]);
         const int n = nc * NO + v * 8;
         const size_t pix = (size_t)(b * a.H + y) * a.W + x;
+        if (n < a.oc0 && a.mask0) val = relu_masked(val, *reinterpret_cast<const uint4*>(&a.mask0[pix * a.oc0 + n]));
         if (n < a.oc0) *reinterpret_cast<uint4*>(&a.out0[pix * a.oc0 + n]) = val;
         else *reinterpret_cast<uint4*>(&a.out1[pix * a.oc1 + (n - a.oc0)]) = val;
     }
@@ -1498,53 +1515,40 @@ __global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__
 }
 
 // ------------------------------------------------------------- weight packing
-// Forward packing: [c][s][n][j] = W[tap][ci][n], K index s*32+j = tap*CC + (ci mod CC).
-__global__ __launch_bounds__(256) void k_pack_fwd(const float* __restrict__ w, uint16_t* __restrict__ wf, int cin,
-                                                  int cout, int np, int CC, int KS, int total) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int j = idx & 31;
-    const int n = (idx >> 5) % np;
-    const int s = (idx / (32 * np)) % KS;
-    const int c = idx / (32 * np * KS);
-    const int kf = s * 32 + j;
-    const int tap = kf / CC, ci = c * CC + (kf - tap * CC);
-    float v = 0.0f;
-    if (tap < 9 && n < cout && ci < cin) v = w[((size_t)tap * cin + ci) * cout + n];
-    wf[idx] = f2bf(v);
-}
+// One layer's packed copy: forward, [c][s][n][j] = W[tap][ci][n], K index s*32+j =
+// tap*CC + (ci mod CC); or the input gradient's, a forward convolution over the output
+// gradient with W'[t][co][ci] = W[8-t][ci][co] in chunks of 32 over cout (padded).
+struct PackJob {
+    const float* w;
+    uint16_t* out;
+    int cin, cout, np, cc, ks, dgrad, total, block0;   // np: outputs (forward) or cin; first block
+};
+constexpr int kMaxPackJobs = 40;
+struct PackJobs {
+    int n;
+    PackJob job[kMaxPackJobs];
+};
 
-// Input-gradient packing: a forward convolution over the output gradient with
-// W'[t][co][ci] = W[8-t][ci][co]; chunks of 32 over cout (padded to np).
-__global__ __launch_bounds__(256) void k_pack_dgrad(const float* __restrict__ w, uint16_t* __restrict__ wd, int cin,
-                                                    int cout, int total) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int j = idx & 31;
-    const int n = (idx >> 5) % cin;
-    const int s = (idx / (32 * cin)) % 9;
-    const int c = idx / (32 * cin * 9);
-    const int co = c * 32 + j;
+// All layers' copies in one launch, 34 us; 37 launches of 2 to 3 us each took 114 us of a step.
+__global__ __launch_bounds__(256) void k_pack(PackJobs jobs) {
+    int k = 0;
+    while (k + 1 < jobs.n && (int)blockIdx.x >= jobs.job[k + 1].block0) ++k;   // uniform
+    const PackJob& J = jobs.job[k];
+    const int idx = ((int)blockIdx.x - J.block0) * 256 + threadIdx.x;
+    if (idx >= J.total) return;
+    const int j = idx & 31, n = (idx >> 5) % J.np, s = (idx / (32 * J.np)) % J.ks, c = idx / (32 * J.np * J.ks);
     float v = 0.0f;
-    if (co < cout) v = w[((size_t)(8 - s) * cin + n) * cout + co];
-    wd[idx] = f2bf(v);
+    if (J.dgrad) {
+        const int co = c * 32 + j;
+        if (co < J.cout) v = J.w[((size_t)(8 - s) * J.cin + n) * J.cout + co];
+    } else {
+        const int kf = s * 32 + j, tap = kf / J.cc, ci = c * J.cc + (kf - tap * J.cc);
+        if (tap < 9 && n < J.cout && ci < J.cin) v = J.w[((size_t)tap * J.cin + ci) * J.cout + n];
+    }
+    J.out[idx] = f2bf(v);
 }
 
 // ------------------------------------------------------- elementwise kernels
-__global__ __launch_bounds__(256) void k_relu_mask(uint16_t* __restrict__ g, const uint16_t* __restrict__ y,
-                                                   size_t n8) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n8) return;
-    uint4 gv = reinterpret_cast<uint4*>(g)[i];
-    const uint4 yv = reinterpret_cast<const uint4*>(y)[i];
-    uint16_t* ge = reinterpret_cast<uint16_t*>(&gv);
-    const uint16_t* ye = reinterpret_cast<const uint16_t*>(&yv);
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        if (!(bf2f(ye[k]) > 0.0f)) ge[k] = 0;
-    reinterpret_cast<uint4*>(g)[i] = gv;
-}
-
 // 2x2 max-pool, H and W even.
 __global__ __launch_bounds__(256) void k_pool_fwd(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int B,
                                                   int H, int W, int C) {
@@ -1567,10 +1571,10 @@ __global__ __launch_bounds__(256) void k_pool_fwd(const uint16_t* __restrict__ i
 }
 
 // Routes the pooled gradient to the first maximum of each 2x2 window (scan
-// order (0,0),(0,1),(1,0),(1,1)); adds into gin when accumulate != 0.
+// order (0,0),(0,1),(1,0),(1,1)), adds it to gin (the skip's gradient) and zeroes the
+// sum where the ReLU output `in` is not positive.
 __global__ __launch_bounds__(256) void k_pool_bwd(const uint16_t* __restrict__ in, const uint16_t* __restrict__ gout,
-                                                  uint16_t* __restrict__ gin, int accumulate, int B, int H, int W,
-                                                  int C) {
+                                                  uint16_t* __restrict__ gin, int B, int H, int W, int C) {
     const int h = H >> 1, w = W >> 1, cv = C >> 3;
     // 32-bit index arithmetic: check_shape bounds B*Hp*Wp by 2^28, so B*h*w*cv < 2^32
     const uint32_t total = (uint32_t)B * h * w * cv;
@@ -1588,7 +1592,7 @@ __global__ __launch_bounds__(256) void k_pool_bwd(const uint16_t* __restrict__ i
     for (int k = 0; k < 4; ++k) {
         off[k] = ((size_t)(b * H + 2 * y + (k >> 1)) * W + 2 * x + (k & 1)) * C + v * 8;
         q[k] = *reinterpret_cast<const uint4*>(in + off[k]);
-        gi[k] = accumulate ? *reinterpret_cast<const uint4*>(gin + off[k]) : make_uint4(0u, 0u, 0u, 0u);
+        gi[k] = *reinterpret_cast<const uint4*>(gin + off[k]);
     }
     const uint4 go = *reinterpret_cast<const uint4*>(gout + ((size_t)(b * h + y) * w + x) * C + v * 8);
 #pragma unroll
@@ -1604,7 +1608,7 @@ __global__ __launch_bounds__(256) void k_pool_bwd(const uint16_t* __restrict__ i
         t[e] = f2bf(bf2f(t[e]) + bf2f(reinterpret_cast<const uint16_t*>(&go)[e]));
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) *reinterpret_cast<uint4*>(gin + off[k]) = gi[k];
+    for (int k = 0; k < 4; ++k) *reinterpret_cast<uint4*>(gin + off[k]) = relu_masked(gi[k], q[k]);
 }
 
 __global__ __launch_bounds__(256) void k_up_fwd(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int B,
@@ -1633,9 +1637,9 @@ __device__ inline float up_weight(int X, int n, int i) {
 }
 
 // Transpose of k_up_fwd in gather form (each input sample sums the output
-// samples that read it, fixed order).
-__global__ __launch_bounds__(256) void k_up_bwd(const uint16_t* __restrict__ gout, uint16_t* __restrict__ gin, int B,
-                                                int h, int w, int C) {
+// samples that read it, fixed order), zeroed where the ReLU output `in` is not positive.
+__global__ __launch_bounds__(256) void k_up_bwd(const uint16_t* __restrict__ gout, const uint16_t* __restrict__ in,
+                                                uint16_t* __restrict__ gin, int B, int h, int w, int C) {
     const int H = 2 * h, W = 2 * w, cv = C >> 3;
     // 32-bit index arithmetic: check_shape bounds B*Hp*Wp by 2^28, so B*h*w*cv < 2^32
     const uint32_t total = (uint32_t)B * h * w * cv;
@@ -1664,7 +1668,8 @@ __global__ __launch_bounds__(256) void k_up_bwd(const uint16_t* __restrict__ gou
     uint16_t* oe = reinterpret_cast<uint16_t*>(&o);
 #pragma unroll
     for (int e = 0; e < 8; ++e) oe[e] = f2bf(acc[e]);
-    *reinterpret_cast<uint4*>(gin + ((size_t)(b * h + y) * w + x) * C + v * 8) = o;
+    const size_t at = ((size_t)(b * h + y) * w + x) * C + v * 8;
+    *reinterpret_cast<uint4*>(gin + at) = relu_masked(o, *reinterpret_cast<const uint4*>(in + at));
 }
 
 // Guide images -> 16-channel bf16 input at padded size (edge replication):
@@ -2004,6 +2009,9 @@ void conv_dgrad(ohpt_denoiser* d, const Layer& L, const uint16_t* G, int lvl) {
     a.np = L.cin;
     a.out0 = d->gact[L.sp.in0].as<uint16_t>();
     a.oc0 = L.cin0;
+    // pooled and upsampled inputs are no ReLU outputs: what they lead to is masked there
+    static constexpr bool kRelu[kNumAct] = {0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1};
+    a.mask0 = kRelu[L.sp.in0] ? d->act[L.sp.in0].as<uint16_t>() : nullptr;
     a.out1 = L.sp.in1 >= 0 ? d->gact[L.sp.in1].as<uint16_t>() : nullptr;
     a.oc1 = L.cin1;
     a.B = d->B;
@@ -2050,11 +2058,6 @@ hipError_t conv_wgrad(ohpt_denoiser* d, const Layer& L, const uint16_t* G, int l
     return hipSuccess;
 }
 
-void relu_mask(ohpt_denoiser* d, int t) {
-    const size_t n = ((size_t)d->B * d->Hp * d->Wp >> (2 * kActLevel[t])) * kActChan[t];
-    k_relu_mask<<<cdiv(n / 8, 256), 256, 0, d->stream>>>(d->gact[t].as<uint16_t>(), d->act[t].as<uint16_t>(), n / 8);
-}
-
 void pool_forward(ohpt_denoiser* d, int src, int dst) {
     const int lvl = kActLevel[src], C = kActChan[src];
     const int H = d->Hp >> lvl, W = d->Wp >> lvl;
@@ -2068,7 +2071,7 @@ void pool_backward(ohpt_denoiser* d, int src, int dst) {   // dst = pooled tenso
     const int H = d->Hp >> lvl, W = d->Wp >> lvl;
     const size_t n = (size_t)d->B * (H / 2) * (W / 2) * (C / 8);
     k_pool_bwd<<<cdiv(n, 256), 256, 0, d->stream>>>(d->act[src].as<uint16_t>(), d->gact[dst].as<uint16_t>(),
-                                                    d->gact[src].as<uint16_t>(), 1, d->B, H, W, C);
+                                                    d->gact[src].as<uint16_t>(), d->B, H, W, C);
 }
 
 void up_forward(ohpt_denoiser* d, int src, int dst) {
@@ -2083,8 +2086,8 @@ void up_backward(ohpt_denoiser* d, int src, int dst) {   // gradient of dst (ups
     const int lvl = kActLevel[src], C = kActChan[src];
     const int h = d->Hp >> lvl, w = d->Wp >> lvl;
     const size_t n = (size_t)d->B * h * w * (C / 8);
-    k_up_bwd<<<cdiv(n, 256), 256, 0, d->stream>>>(d->gact[dst].as<uint16_t>(), d->gact[src].as<uint16_t>(), d->B, h,
-                                                  w, C);
+    k_up_bwd<<<cdiv(n, 256), 256, 0, d->stream>>>(d->gact[dst].as<uint16_t>(), d->act[src].as<uint16_t>(),
+                                                  d->gact[src].as<uint16_t>(), d->B, h, w, C);
 }
 
 double conv_flops(const ohpt_denoiser* d, int H, int W, bool training) {
@@ -2143,7 +2146,8 @@ void network_forward(ohpt_denoiser* d, bool training, const FeatureSrc& feat, fl
     }
 }
 
-// Backward of one ReLU convolution given the gradient of its output tensor.
+// Backward of one convolution given the gradient of its output tensor, which the
+// kernel that wrote it last has masked by the ReLU (k_up_bwd, k_pool_bwd, conv_dgrad).
 hipError_t layer_backward(ohpt_denoiser* d, int li, bool need_input_grad) {
     const Layer& L = d->layers[li];
     const int lvl = kActLevel[L.sp.in0];
@@ -2151,7 +2155,6 @@ hipError_t layer_backward(ohpt_denoiser* d, int li, bool need_input_grad) {
     if (L.sp.out == kLogits) {
         G = d->dlogits.as<uint16_t>();
     } else {
-        relu_mask(d, L.sp.out);
         G = d->gact[L.sp.out].as<uint16_t>();
     }
     hipError_t e = conv_wgrad(d, L, G, lvl);
@@ -2194,15 +2197,18 @@ hipError_t network_backward(ohpt_denoiser* d) {
 }
 
 hipError_t pack_weights(ohpt_denoiser* d) {
-    for (Layer& L : d->layers) {
-        const float* w = d->params.as<float>() + L.w_off;
-        const int nf = L.nchunk * L.ks * L.np * 32;
-        k_pack_fwd<<<cdiv(nf, 256), 256, 0, d->stream>>>(w, L.wf.as<uint16_t>(), L.cin, L.cout, L.np, L.cc, L.ks, nf);
-        if (L.sp.in0 != X0) {
-            const int nd = (L.np / 32) * 9 * L.cin * 32;
-            k_pack_dgrad<<<cdiv(nd, 256), 256, 0, d->stream>>>(w, L.wd.as<uint16_t>(), L.cin, L.cout, nd);
-        }
+    PackJobs P{};
+    static_assert(2 * kNumLayers <= kMaxPackJobs, "a forward and an input-gradient copy per layer");
+    int blocks = 0;
+    auto add = [&](const Layer& L, uint16_t* out, int np, int cc, int ks, int dgrad, int total) {
+        P.job[P.n++] = PackJob{d->params.as<float>() + L.w_off, out, L.cin, L.cout, np, cc, ks, dgrad, total, blocks};
+        blocks += (int)cdiv(total, 256);
+    };
+    for (const Layer& L : d->layers) {
+        add(L, L.wf.as<uint16_t>(), L.np, L.cc, L.ks, 0, L.nchunk * L.ks * L.np * 32);
+        if (L.sp.in0 != X0) add(L, L.wd.as<uint16_t>(), L.cin, 32, 9, 1, (L.np / 32) * 9 * L.cin * 32);
     }
+    k_pack<<<blocks, 256, 0, d->stream>>>(P);
     return hipGetLastError();
 }
 
