@@ -621,6 +621,8 @@ __device__ __align__(16) uint32_t g_zero_vec[4] = {0u, 0u, 0u, 0u};
 // 16-byte slot 64 i + l, so each lane fetches the vector that the XOR-swizzled
 // layouts of k_conv3x3 keep in that slot. The MFMA order per accumulator
 // (chunks, then K steps) and the epilogue are k_conv3x3's: bit-identical outputs.
+// kMask: an input gradient with a ReLU mask (a.mask0); the other layers run without its test.
+template <bool kMask>
 __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
     constexpr int CC = 32, RW = 16, TX = 16, NT = 512, NO = 32, KS = 9;
     constexpr int HX = TX + 2, HP = HX * (RW + 2);   // 18 x 18 halo pixels
@@ -766,7 +768,7 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
         uint4 val = *reinterpret_cast<const uint4*>(&os[pl * OS + v * 8]);
         const int n = nc * NO + v * 8;
         const size_t pix = (size_t)(b * a.H + y) * a.W + x;
-        if (n < a.oc0 && a.mask0) val = relu_masked(val, *reinterpret_cast<const uint4*>(&a.mask0[pix * a.oc0 + n]));
+        if (kMask && n < a.oc0) val = relu_masked(val, *reinterpret_cast<const uint4*>(&a.mask0[pix * a.oc0 + n]));
         if (n < a.oc0) *reinterpret_cast<uint4*>(&a.out0[pix * a.oc0 + n]) = val;
         else *reinterpret_cast<uint4*>(&a.out1[pix * a.oc1 + (n - a.oc0)]) = val;
     }
@@ -1940,7 +1942,8 @@ void launch_conv(ohpt_denoiser* d, const Layer& L, const ConvArgs& a, int cc) {
         const int64_t slots = 2ll * d->num_cus, work = (int64_t)n_tiles * ncout;
         if (work <= 2 * slots) {
             grid.z = (uint32_t)(a.B * ncout);
-            k_conv_dma<<<grid, 512, 0, d->stream>>>(a);
+            if (a.mask0) k_conv_dma<true><<<grid, 512, 0, d->stream>>>(a);
+            else k_conv_dma<false><<<grid, 512, 0, d->stream>>>(a);
         } else {
             p.per_block = work < 3 * slots - ncout ? 1 : (int)cdiv(n_tiles, (uint64_t)std::max<int64_t>(1, slots / ncout));
             k_conv_ring<<<(cdiv(n_tiles, p.per_block) * ncout + 7u) & ~7u, 512, 0, d->stream>>>(p);
