@@ -118,7 +118,7 @@ struct ohpt_context {
     // path state
     uint32_t capacity = 0;
     DevBuf ps_o, ps_d, ps_T, ps_L, ps_ln0, ps_ln1, ps_aov0, ps_aov1, ps_q0, ps_q1, ps_hits, sh_o, sh_d, sh_c,
-        counters, fetch, ovf, tmp, tstats;
+        counters, ovf, tmp, tstats;   // ovf: stack slots, then fetch counters
     uint32_t ovf_rays = 0;
     DevBuf adj_vis, adj_lrem, adj_dldi, adj_hits;   // path-replay adjoint state
     DevBuf rec_key2, rec_val2, rec_count, rec_tiles; // deterministic mode: compacted records
@@ -221,11 +221,8 @@ int alloc_frame(ohpt_context* c) {
 
 int clear_frame(ohpt_context* c) {
     const size_t npix = (size_t)c->W * c->H;
-    launch_fill_u32(c->d_accum.as<uint32_t>(), 0u, (uint32_t)(npix * 4), c->stream);
-    launch_fill_u32(c->d_moments.as<uint32_t>(), 0u, (uint32_t)(npix * 4), c->stream);
-    launch_fill_u32(c->d_aov_albedo.as<uint32_t>(), 0u, (uint32_t)(npix * 4), c->stream);
-    launch_fill_u32(c->d_aov_normal.as<uint32_t>(), 0u, (uint32_t)(npix * 4), c->stream);
-    launch_fill_u32(c->d_disp.as<uint32_t>(), 0u, (uint32_t)(npix * 4), c->stream);
+    launch_clear_frame(c->d_accum.as<float4>(), c->d_moments.as<float4>(), c->d_aov_albedo.as<float4>(),
+                       c->d_aov_normal.as<float4>(), c->d_disp.as<float4>(), (uint32_t)npix, c->stream);
     HIPCHK(hipGetLastError());
     c->reference_samples = false;
     return OHPT_OK;
@@ -241,13 +238,14 @@ int need_guides(const ohpt_context* c, const char* what) {
     return OHPT_OK;
 }
 
-// Stack overflow slots and fetch counters of the traversals, for every lane: one size
-// for the context's life, so they are never replaced under a launch in flight.
+// Stack overflow slots and fetch counters of the traversals, for every lane, in one
+// allocation: one size for the context's life, so it is never replaced under a launch
+// in flight.
+size_t ovf_bytes() { return trace_overflow_bytes() * ohpt_context::kLanes; }
 hipError_t ensure_trace_scratch(ohpt_context* c) {
-    const hipError_t e = c->ovf.ensure(trace_overflow_bytes() * ohpt_context::kLanes);
-    return e != hipSuccess ? e
-                           : c->fetch.ensure((size_t)kFetchWords * kMaxTraceLaunches * 4 * ohpt_context::kLanes);
+    return c->ovf.ensure(ovf_bytes() + (size_t)kFetchWords * kMaxTraceLaunches * 4 * ohpt_context::kLanes);
 }
+uint32_t* trace_fetch(ohpt_context* c) { return c->ovf.as<uint32_t>() + ovf_bytes() / 4; }
 
 int ensure_paths(ohpt_context* c, uint32_t n) {
     if (n <= c->capacity) return OHPT_OK;
@@ -317,7 +315,7 @@ PathState path_state(ohpt_context* c, int set = 0) {
     p.sh_d = c->sh_d.as<float4>();
     p.sh_c = c->sh_c.as<float4>();
     p.counters = c->counters.as<uint32_t>();
-    p.fetch = c->fetch.as<uint32_t>();
+    p.fetch = trace_fetch(c);
     p.capacity = c->capacity;
     return p;
 }
@@ -1863,7 +1861,7 @@ int ray_batch(ohpt_context* c, const float* rays, void* out, uint32_t n, int on_
         o = dout.p;
     }
     const DevScene S = scene_view(c);
-    uint32_t* const fetch = c->fetch.as<uint32_t>();
+    uint32_t* const fetch = trace_fetch(c);
     uint32_t* const ovf = c->ovf.as<uint32_t>();
     if (occl) launch_occluded_rays(S, r, reinterpret_cast<uint32_t*>(o), n, fetch, ovf, c->stream);
     else launch_trace_rays(S, r, reinterpret_cast<float4*>(o), n, fetch, ovf, c->stream);

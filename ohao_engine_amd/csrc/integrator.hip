@@ -29,6 +29,15 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint32_t n) {
     if (i < n) p[i] = v;
 }
 
+// The five accumulation buffers of a frame in one launch of 16-byte stores (five fills of
+// 4-byte stores: 45 us at 1920x1080 and four more launches).
+__global__ __launch_bounds__(256) void k_clear_frame(float4* a, float4* b, float4* c, float4* d, float4* e, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    a[i] = z; b[i] = z; c[i] = z; d[i] = z; e[i] = z;
+}
+
 __global__ __launch_bounds__(256) void k_clear_counters(uint32_t* counters, uint32_t* fetch, uint32_t nfetch) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < kCounterWords) counters[i] = 0u;
@@ -563,6 +572,10 @@ inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) /
 
 void launch_fill_u32(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s) {
     if (n) k_fill_u32<<<div_up(n, 256), 256, 0, s>>>(p, v, n);
+}
+
+void launch_clear_frame(float4* a, float4* b, float4* c, float4* d, float4* e, uint32_t n, hipStream_t s) {
+    if (n) k_clear_frame<<<div_up(n, 256), 256, 0, s>>>(a, b, c, d, e, n);
 }
 
 void launch_clear_counters(const PathState& ps, uint32_t launches, hipStream_t s) {

@@ -164,6 +164,8 @@ static_assert(sh_counter(62) < kCounterWords && kCounterWords % 2 == 0, "counter
 inline uint32_t* fetch_counters(const PathState& ps, uint32_t b) { return ps.fetch + (size_t)b * kFetchWords; }
 // Zeroes the queue lengths and the fetch counters of the batch's first `launches` traversals.
 void launch_clear_counters(const PathState& ps, uint32_t launches, hipStream_t s);
+// Zeroes n float4 of each of five buffers.
+void launch_clear_frame(float4* a, float4* b, float4* c, float4* d, float4* e, uint32_t n, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t v, uint32_t n, hipStream_t s);
 void launch_generate(const FrameParams& f, const PathState& ps, hipStream_t s);
 void launch_shade(const DevScene& S, const FrameParams& f, const PathState& ps, uint32_t bounce, hipStream_t s);
