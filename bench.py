@@ -260,7 +260,7 @@ def denoise_leg(ctx, sc, ref_spp, save_dir=None):
            "gate": {"enabled": gate.enabled, "bound": gate.bound},
            "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": BF16_PEAK_TFLOPS,
                         "unit": "TFLOP/s", "frac": round(achieved / BF16_PEAK_TFLOPS, 5),
-                        "kernel": "k_conv_stream (4 full-resolution layers) + k_conv_dma (11 layers at levels "
+                        "kernel": "k_conv_features + k_conv_stream (4 full-resolution layers) + k_conv_ring, k_conv_dma (11 layers at levels "
                                   "1-4) + k_conv3x3 (4 upsampling decoder layers): BF16 MFMA implicit GEMM, "
                                   "19 convolutions",
                         "conv_gflop_per_inference": round(conv_flops / 1e9, 2), "conv_ms": round(ms_conv, 3),
