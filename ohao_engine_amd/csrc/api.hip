@@ -42,13 +42,22 @@ namespace {
         if (e_ != hipSuccess) return fail_hip(#x, e_); \
     } while (0)
 
+// Waits for the stream where a call returns early, so that no copy enqueued so far still
+// reads or writes host memory that the call or its caller owns.
+struct WaitOnError {
+    hipStream_t stream;
+    bool armed = true;
+    ~WaitOnError() {
+        if (armed) (void)hipStreamSynchronize(stream);
+    }
+};
+
 struct TexStore {
     DevBuf data;
     uint32_t w = 0, h = 0, c = 0;
     double mean[3] = {0, 0, 0};   // mean texel per channel as sampled (one channel reads as grey)
     size_t packed_floats() const { return (size_t)w * h * (c >= 2 ? 4u : 1u); }
 };
-
 
 }  // namespace
 
@@ -784,6 +793,9 @@ int ohpt_scene_commit(ohpt_context* c) {
         c->n_nodes4 = 0;
         return build_emitters(c);
     }
+    // the copies read the runs and the staged meshes until the stream has been waited for
+    std::deque<MeshRun> runs;
+    WaitOnError wait{c->stream};
     // the world-space triangles stay resident for refits
     DevBuf& pos = c->d_tpos;
     DevBuf& nrm = c->d_tnrm;
@@ -798,7 +810,6 @@ int ohpt_scene_commit(ohpt_context* c) {
     if (c->any_uv) {
         HIPCHK(uv.ensure((size_t)n * 24));
     }
-    std::deque<MeshRun> runs;   // the copies read them until the build has waited for the stream
     for (size_t i = 0; i < c->meshes.size();) {
         if (c->meshes[i].nt >= kHostMeshTriangles) {
             if (int r = place_mesh(c, c->meshes[i++])) return r;
@@ -842,6 +853,7 @@ int ohpt_scene_commit(ohpt_context* c) {
     if (e != hipSuccess) return fail_hip("bvh4_collapse", e);
     HIPCHK(hipEventRecord(c->ev_stop, c->stream));
     HIPCHK(hipEventSynchronize(c->ev_stop));
+    wait.armed = false;
     c->stats.ms_build = elapsed(c->ev_start, c->ev_stop);
     c->n_nodes4 = n4;
     c->committed = true;

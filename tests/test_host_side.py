@@ -1,0 +1,70 @@
+"""What the library's host side leaves behind, watched without a GPU: the library runs in a
+process of its own over tests/hip_recorder.cpp, which takes the HIP runtime's place, runs no
+kernel, and counts copies that nothing has waited for and bytes that are allocated."""
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+
+PRELUDE = """
+import ctypes as C, sys
+sys.modules["torch"] = None                    # its own copy of the runtime stays out of this process
+R = C.CDLL({recorder!r}, mode=C.RTLD_GLOBAL)   # found before the runtime that the library links
+R.rec_allocated.restype = R.rec_peak.restype = C.c_size_t
+R.rec_fail_malloc.argtypes = R.rec_fail_copy.argtypes = [C.c_long]
+R.rec_launch.restype = C.c_char_p
+sys.path.insert(0, {root!r})
+import numpy as np
+from ohao_engine_amd import ohpt, scenes as S
+
+def launches():
+    g = (C.c_uint32 * 3)()
+    return [(R.rec_launch(i, g).decode(), tuple(g)) for i in range(R.rec_launches())]
+"""
+
+
+@pytest.fixture(scope="module")
+def recorded(tmp_path_factory):
+    lib = tmp_path_factory.mktemp("recorder") / "libhip_recorder.so"
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", str(lib), str(ROOT / "tests" / "hip_recorder.cpp")],
+                   check=True)
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRELUDE.format(recorder=str(lib), root=str(ROOT)) + code],
+                           capture_output=True, text=True, timeout=300)
+        assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-4000:]
+        return p.stdout
+
+    return run
+
+
+@pytest.mark.parametrize("what", ["malloc", "copy"])
+def test_a_failed_commit_leaves_no_copy_in_flight(recorded, what):
+    """Small meshes are expanded into host arrays that the call owns: whichever allocation or
+    copy of the commit fails, no copy may still read them when it returns."""
+    out = recorded(f"""
+failed, left = 0, []
+for n in range(60):
+    ctx = ohpt.Context(16, 16)
+    ctx.begin_scene()
+    rng = np.random.default_rng(0)
+    for nt, world in ((7, None), (3000, 2 * np.eye(4)), (5, None), (2500, None), (4, None)):
+        v = rng.random((nt + 2, 3), dtype=np.float32)
+        ctx.add_mesh(v, rng.integers(0, nt + 2, (nt, 3)), normals=v, world=world)
+    R.rec_fail_{what}(n)
+    rc = ctx.L.ohpt_scene_commit(ctx.h)
+    R.rec_fail_{what}(-1)
+    if rc == 0:
+        break
+    failed += 1
+    if R.rec_pending():
+        left.append((n, R.rec_pending()))
+    ctx.close()
+print(rc, failed, left)
+""")
+    rc, failures, left = out.strip().split(" ", 2)
+    assert int(rc) == 0 and int(failures) >= 10      # every one of them failed once, then none
+    assert left == "[]", f"(failing one, copies in flight): {left}"
