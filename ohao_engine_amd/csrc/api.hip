@@ -994,6 +994,7 @@ int fill_texture(ohpt_context* c, TexStore& t, const float* texels, int on_devic
     const size_t mean_at = (bytes + 15) & ~size_t(15);
     HIPCHK(t.data.ensure(t.packed_floats() * 4));
     HIPCHK(c->tmp.ensure(mean_at + texel_mean_scratch_bytes()));
+    WaitOnError wait{c->stream};
     if (on_device) {
         HIPCHK(hipMemcpy(c->tmp.p, texels, bytes, hipMemcpyDefault));
         HIPCHK(hipStreamSynchronize(nullptr));
@@ -1004,6 +1005,7 @@ int fill_texture(ohpt_context* c, TexStore& t, const float* texels, int on_devic
     launch_texel_pack(c->tmp.as<float>(), n, t.c, t.data.as<float>(), mean, c->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(t.mean, mean, sizeof t.mean, hipMemcpyDeviceToHost, c->stream));
+    wait.armed = false;
     HIPCHK(hipStreamSynchronize(c->stream));
     return OHPT_OK;
 }

@@ -68,3 +68,29 @@ print(rc, failed, left)
     rc, failures, left = out.strip().split(" ", 2)
     assert int(rc) == 0 and int(failures) >= 10      # every one of them failed once, then none
     assert left == "[]", f"(failing one, copies in flight): {left}"
+
+
+def test_a_failed_texture_upload_leaves_no_copy_in_flight(recorded):
+    """The texels are the caller's, who may free them as soon as the call returns."""
+    out = recorded("""
+failed, left = 0, []
+for update in (False, True):
+    for n in range(10):
+        ctx = ohpt.Context(16, 16)
+        t = np.ones((5, 7, 3), np.float32)
+        if update:
+            ctx.upload_texture(t)
+        R.rec_fail_copy(n)
+        try:
+            ctx.update_texture(0, t) if update else ctx.upload_texture(t)
+        except ohpt.OhptError:
+            failed += 1
+            if R.rec_pending():
+                left.append((update, n, R.rec_pending()))
+        R.rec_fail_copy(-1)
+        ctx.close()
+print(failed, left)
+""")
+    failures, left = out.strip().split(" ", 1)
+    assert int(failures) >= 4
+    assert left == "[]", f"(update, failing copy, copies in flight): {left}"
