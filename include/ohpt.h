@@ -322,7 +322,10 @@ int ohpt_read_texture_gradient(ohpt_context* ctx, int32_t id, float* out, int on
 /* Trace a batch of caller-supplied rays (closest hit). rays: n x 8 floats
  * (ox,oy,oz,tmin, dx,dy,dz,tmax); hits: n x 4 (t, prim as uint bits, u, v),
  * prim = 0xFFFFFFFF on miss. prim is the caller's global triangle numbering
- * (mesh order, then triangle order). Device pointers when on_device != 0. */
+ * (mesh order, then triangle order). Device pointers when on_device != 0. The
+ * first query allocates the traversal's stack slots, which the context keeps
+ * (about 100 MB on a 256-CU device); renders keep three times as many and
+ * queries share them. */
 int ohpt_trace_rays(ohpt_context* ctx, const float* rays, float* hits, uint32_t n, int on_device);
 /* Occlusion query: out[i] = 1 if any hit in (tmin, tmax). */
 int ohpt_occluded_rays(ohpt_context* ctx, const float* rays, uint32_t* out, uint32_t n, int on_device);

@@ -127,7 +127,7 @@ struct ohpt_context {
     // path state
     uint32_t capacity = 0;
     DevBuf ps_o, ps_d, ps_T, ps_L, ps_ln0, ps_ln1, ps_aov0, ps_aov1, ps_q0, ps_q1, ps_hits, sh_o, sh_d, sh_c,
-        counters, ovf, tmp, tstats;   // ovf: stack slots, then fetch counters
+        counters, ovf, tmp, tstats;   // ovf: fetch counters, then stack slots
     uint32_t ovf_rays = 0;
     DevBuf adj_vis, adj_lrem, adj_dldi, adj_hits;   // path-replay adjoint state
     DevBuf rec_key2, rec_val2, rec_count, rec_tiles; // deterministic mode: compacted records
@@ -247,14 +247,15 @@ int need_guides(const ohpt_context* c, const char* what) {
     return OHPT_OK;
 }
 
-// Stack overflow slots and fetch counters of the traversals, for every lane, in one
-// allocation: one size for the context's life, so it is never replaced under a launch
-// in flight.
-size_t ovf_bytes() { return trace_overflow_bytes() * ohpt_context::kLanes; }
-hipError_t ensure_trace_scratch(ohpt_context* c) {
-    return c->ovf.ensure(ovf_bytes() + (size_t)kFetchWords * kMaxTraceLaunches * 4 * ohpt_context::kLanes);
+// Fetch counters of the traversals (every lane's), then the stack overflow slots of the
+// first `lanes` lanes, in one allocation that only grows: from the one lane of a ray query,
+// which waits for its traversal, to every lane of a render or an adjoint, in ensure_paths,
+// which waits for all streams first. So it is never replaced under a launch in flight.
+constexpr size_t kTraceFetchWords = (size_t)kFetchWords * kMaxTraceLaunches * ohpt_context::kLanes;
+hipError_t ensure_trace_scratch(ohpt_context* c, int lanes) {
+    return c->ovf.ensure(kTraceFetchWords * 4 + trace_overflow_bytes() * (size_t)lanes);
 }
-uint32_t* trace_fetch(ohpt_context* c) { return c->ovf.as<uint32_t>() + ovf_bytes() / 4; }
+uint32_t* trace_fetch(ohpt_context* c) { return c->ovf.as<uint32_t>(); }
 
 int ensure_paths(ohpt_context* c, uint32_t n) {
     if (n <= c->capacity) return OHPT_OK;
@@ -279,7 +280,7 @@ int ensure_paths(ohpt_context* c, uint32_t n) {
     HIPCHK(c->sh_d.ensure(2 * N * 16));
     HIPCHK(c->sh_c.ensure(2 * N * 16));
     HIPCHK(c->counters.ensure((size_t)kCounterWords * 4 * ohpt_context::kLanes));
-    HIPCHK(ensure_trace_scratch(c));
+    HIPCHK(ensure_trace_scratch(c, ohpt_context::kLanes));
     c->ovf_rays = 2 * n;
     c->capacity = n;
     return OHPT_OK;
@@ -302,7 +303,7 @@ PathState lane_view(const PathState& ps, uint32_t pid_base, int lane) {
 }
 
 uint32_t* lane_ovf(ohpt_context* c, int lane) {
-    return c->ovf.as<uint32_t>() + (size_t)lane * (trace_overflow_bytes() / 4);
+    return c->ovf.as<uint32_t>() + kTraceFetchWords + (size_t)lane * (trace_overflow_bytes() / 4);
 }
 
 // set: which copy of the arrays the accumulation reads (0 or 1)
@@ -1863,7 +1864,7 @@ int ray_batch(ohpt_context* c, const float* rays, void* out, uint32_t n, int on_
     if (n == 0) return OHPT_OK;
     HIPCHK(enter(c));
     DevBuf dr, dout;
-    HIPCHK(ensure_trace_scratch(c));
+    HIPCHK(ensure_trace_scratch(c, 1));
     const float4* r = reinterpret_cast<const float4*>(rays);
     void* o = out;
     const size_t out_bytes = (size_t)n * (occl ? 4 : 16);
@@ -1876,7 +1877,7 @@ int ray_batch(ohpt_context* c, const float* rays, void* out, uint32_t n, int on_
     }
     const DevScene S = scene_view(c);
     uint32_t* const fetch = trace_fetch(c);
-    uint32_t* const ovf = c->ovf.as<uint32_t>();
+    uint32_t* const ovf = lane_ovf(c, 0);
     if (occl) launch_occluded_rays(S, r, reinterpret_cast<uint32_t*>(o), n, fetch, ovf, c->stream);
     else launch_trace_rays(S, r, reinterpret_cast<float4*>(o), n, fetch, ovf, c->stream);
     HIPCHK(hipGetLastError());
@@ -1896,7 +1897,7 @@ int ohpt_occluded_rays(ohpt_context* c, const float* rays, uint32_t* out, uint32
 }
 
 // ohpt_trace_rays with device buffers and the per-device `scratch` array in
-// place of the counter and overflow stacks ray_batch allocates: no allocation,
+// place of the context's counters and overflow stacks that ray_batch uses: no allocation,
 // no synchronisation, launches on the context's stream only.
 int ohpt_trace_rays_noalloc(ohpt_context* c, const float* rays, float* hits, uint32_t n) {
     if (!c || (n && (!rays || !hits))) return fail(OHPT_ERR_INVALID_ARG, "ohpt_trace_rays_noalloc: null argument");

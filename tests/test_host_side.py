@@ -94,3 +94,27 @@ print(failed, left)
     failures, left = out.strip().split(" ", 1)
     assert int(failures) >= 4
     assert left == "[]", f"(update, failing copy, copies in flight): {left}"
+
+
+def test_ray_queries_keep_the_scratch_of_one_lane(recorded):
+    """A context that only traces rays runs one traversal at a time; renders run three."""
+    out = recorded("""
+ctx = ohpt.Context(16, 16)
+ctx.begin_scene()
+ctx.add_mesh(np.eye(3, dtype=np.float32), [0, 1, 2])
+ctx.commit_scene()
+rays = np.ones((5, 8), np.float32)
+held = [R.rec_allocated()]
+for call in (ctx.trace_rays, ctx.occluded_rays, ctx.trace_rays):
+    call(rays)
+    held.append(R.rec_allocated() - held[0])
+ctx.render(1)
+ctx.trace_rays(rays)
+held.append(R.rec_allocated() - held[0])
+print(*held[1:])
+""")
+    one, two, three, rendered = map(int, out.split())
+    # the recorder's device holds 256 x 2 blocks of 128 threads, with 72 stack slots of 4 bytes each
+    lane = 256 * 2 * 128 * 72 * 4
+    assert lane <= one < 1.2 * lane and one == two == three
+    assert rendered >= 3 * lane
