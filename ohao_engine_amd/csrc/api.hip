@@ -264,6 +264,7 @@ int ensure_paths(ohpt_context* c, uint32_t n) {
     for (int l = 0; l < ohpt_context::kLanes; ++l) HIPCHK(hipStreamSynchronize(c->lane_stream[l]));
     c->acc_pending[0] = c->acc_pending[1] = false;
     c->stream_dirty = true;
+    c->capacity = 0;   // until every buffer has its new size
     const size_t N = n;
     HIPCHK(c->ps_o.ensure(N * 16));
     HIPCHK(c->ps_d.ensure(N * 16));

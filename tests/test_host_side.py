@@ -118,3 +118,33 @@ print(*held[1:])
     lane = 256 * 2 * 128 * 72 * 4
     assert lane <= one < 1.2 * lane and one == two == three
     assert rendered >= 3 * lane
+
+
+def test_a_render_that_ran_out_of_memory_can_be_followed_by_a_smaller_one(recorded):
+    """Growing the path buffers frees the old ones first: after a failure half way, a render
+    of the old size has to allocate again instead of using what is gone."""
+    out = recorded("""
+bad = []
+for n in range(16):
+    ctx = ohpt.Context(16, 16)
+    ctx.begin_scene()
+    ctx.add_mesh(np.eye(3, dtype=np.float32), [0, 1, 2])
+    ctx.commit_scene()
+    ctx.render(1)
+    before = R.rec_allocated()
+    assert ctx.L.ohpt_resize(ctx.h, 64, 64) == 0
+    grown = R.rec_allocated() - before
+    R.rec_fail_malloc(n)
+    failed = ctx.L.ohpt_render(ctx.h, 1, 0) != 0
+    R.rec_fail_malloc(-1)
+    if not failed:
+        break
+    assert ctx.L.ohpt_resize(ctx.h, 16, 16) == 0
+    ctx.render(1)
+    if R.rec_allocated() < before + grown:
+        bad.append(n)
+    ctx.close()
+print(n, bad)
+""")
+    n, bad = out.strip().split(" ", 1)
+    assert int(n) >= 10 and bad == "[]", out
