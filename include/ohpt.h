@@ -221,7 +221,9 @@ int ohpt_scene_export_bvh(ohpt_context* ctx, void* nodes_out /* (n-1)*64 B */,
 int ohpt_scene_export_bvh4(ohpt_context* ctx, void* nodes4_out, uint32_t capacity, uint32_t* count_out);
 
 /* Materials and textures: updateRTMaterialParams (rt_build.cpp:313-389)
- * rewrites materials without touching the BVH. */
+ * rewrites materials without touching the BVH. Texels (and the vertices of
+ * larger meshes) pass through a device staging buffer, of which the context
+ * keeps up to 256 MB for the next upload. */
 int ohpt_upload_materials(ohpt_context* ctx, const ohpt_material* materials, uint32_t count);
 int ohpt_upload_texture(ohpt_context* ctx, int32_t* out_id, const float* texels,
                         uint32_t width, uint32_t height, uint32_t channels);

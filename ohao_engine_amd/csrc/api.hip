@@ -653,6 +653,13 @@ int ohpt_resize(ohpt_context* c, uint32_t width, uint32_t height) {
 // ---------------------------------------------------------------- scene
 extern "C++" {
 namespace {
+// Staging of this size stays with the context for the next upload; a call that needed more
+// gives it back once its copies and kernels are done.
+constexpr size_t kKeptStaging = 256u << 20;
+void give_back(ohpt_context* c, size_t needed) {
+    if (needed > kKeptStaging) c->tmp.release();
+}
+
 // Runs of meshes below kHostMeshTriangles are expanded on the host: the four
 // copies of a mesh take about as long as this loop over that many triangles, so a scene
 // of many small meshes is uploaded in few copies.
@@ -694,7 +701,8 @@ int place_run(ohpt_context* c, const MeshRun& r) {
 // copied as it is; the others are gathered on the device from their vertices.
 // (Loading the 200,000-triangle lantern, one flat mesh: 5.5 -> 3.9 ms; the host expanded
 // every corner in double, into zeroed arrays, before the copy.)
-int place_mesh(ohpt_context* c, const ohpt_context::MeshRec& m) {
+// staged: grows to the staging bytes it used.
+int place_mesh(ohpt_context* c, const ohpt_context::MeshRec& m, size_t& staged) {
     if (m.nt == 0) return OHPT_OK;
     float* const tpos = c->d_tpos.as<float>() + (size_t)m.base * 9;
     float* const tnrm = c->any_nrm ? c->d_tnrm.as<float>() + (size_t)m.base * 9 : nullptr;
@@ -711,7 +719,9 @@ int place_mesh(ohpt_context* c, const ohpt_context::MeshRec& m) {
     }
     const size_t pb = m.pos.size() * 4, nb = m.nrm.size() * 4, ub = m.uv.size() * 4, ib = corners * 4;
     auto pad = [](size_t b) { return (b + 15) & ~size_t(15); };
-    HIPCHK(c->tmp.ensure(pad(pb) + pad(nb) + pad(ub) + ib));
+    const size_t bytes = pad(pb) + pad(nb) + pad(ub) + ib;
+    staged = std::max(staged, bytes);
+    HIPCHK(c->tmp.ensure(bytes));
     char* const dp = c->tmp.as<char>();
     char* const dn = dp + pad(pb);
     char* const du = dn + pad(nb);
@@ -797,6 +807,7 @@ int ohpt_scene_commit(ohpt_context* c) {
     }
     // the copies read the runs and the staged meshes until the stream has been waited for
     std::deque<MeshRun> runs;
+    size_t staged = 0;
     WaitOnError wait{c->stream};
     // the world-space triangles stay resident for refits
     DevBuf& pos = c->d_tpos;
@@ -814,7 +825,7 @@ int ohpt_scene_commit(ohpt_context* c) {
     }
     for (size_t i = 0; i < c->meshes.size();) {
         if (c->meshes[i].nt >= kHostMeshTriangles) {
-            if (int r = place_mesh(c, c->meshes[i++])) return r;
+            if (int r = place_mesh(c, c->meshes[i++], staged)) return r;
             continue;
         }
         MeshRun& run = runs.emplace_back();
@@ -856,6 +867,7 @@ int ohpt_scene_commit(ohpt_context* c) {
     HIPCHK(hipEventRecord(c->ev_stop, c->stream));
     HIPCHK(hipEventSynchronize(c->ev_stop));
     wait.armed = false;
+    give_back(c, staged);
     c->stats.ms_build = elapsed(c->ev_start, c->ev_stop);
     c->n_nodes4 = n4;
     c->committed = true;
@@ -993,9 +1005,9 @@ namespace {
 // kernels stay ordered behind the context's own renders.
 int fill_texture(ohpt_context* c, TexStore& t, const float* texels, int on_device) {
     const size_t n = (size_t)t.w * t.h, bytes = n * t.c * 4;
-    const size_t mean_at = (bytes + 15) & ~size_t(15);
+    const size_t mean_at = (bytes + 15) & ~size_t(15), staged = mean_at + texel_mean_scratch_bytes();
     HIPCHK(t.data.ensure(t.packed_floats() * 4));
-    HIPCHK(c->tmp.ensure(mean_at + texel_mean_scratch_bytes()));
+    HIPCHK(c->tmp.ensure(staged));
     WaitOnError wait{c->stream};
     if (on_device) {
         HIPCHK(hipMemcpy(c->tmp.p, texels, bytes, hipMemcpyDefault));
@@ -1009,6 +1021,7 @@ int fill_texture(ohpt_context* c, TexStore& t, const float* texels, int on_devic
     HIPCHK(hipMemcpyAsync(t.mean, mean, sizeof t.mean, hipMemcpyDeviceToHost, c->stream));
     wait.armed = false;
     HIPCHK(hipStreamSynchronize(c->stream));
+    give_back(c, staged);
     return OHPT_OK;
 }
 }  // namespace
@@ -1519,6 +1532,7 @@ int ohpt_read_texture_gradient(ohpt_context* c, int32_t id, float* out, int on_d
         HIPCHK(hipMemcpy(out, src, bytes, hipMemcpyDefault));
         HIPCHK(hipStreamSynchronize(nullptr));
     }
+    if (src == c->tmp.as<float>()) give_back(c, bytes);
     return OHPT_OK;
 }
 

@@ -148,3 +148,29 @@ print(n, bad)
 """)
     n, bad = out.strip().split(" ", 1)
     assert int(n) >= 10 and bad == "[]", out
+
+
+def test_staging_of_large_uploads_is_given_back(recorded):
+    """Texels and vertices pass through a staging buffer: up to 256 MB of it stay with the
+    context for the next upload, more is freed before the call returns."""
+    out = recorded("""
+def held(h, w, nv):
+    # a texture upload, its update and a commit: what stays allocated beyond the texture and the scene
+    ctx = ohpt.Context(16, 16)
+    ctx.begin_scene()
+    ctx.add_mesh(np.zeros((nv, 3), np.float32), np.arange(3 * 2048)[::-1] % nv)
+    before = R.rec_allocated()
+    ctx.commit_scene()
+    scene = R.rec_allocated() - before
+    t = np.zeros((h, w, 3), np.float32)
+    before = R.rec_allocated()
+    ctx.upload_texture(t)
+    ctx.update_texture(0, t)
+    texture = R.rec_allocated() - before - h * w * 16
+    ctx.close()
+    return scene, texture
+print(*held(8, 8, 3 * 2048), *held(4800, 4800, 24 << 20))
+""")
+    scene, texture, large_scene, large_texture = map(int, out.split())
+    assert abs(large_scene - scene) < (1 << 20), (scene, large_scene)
+    assert abs(large_texture - texture) < (1 << 20), (texture, large_texture)
