@@ -1932,9 +1932,14 @@ void launch_conv(ohpt_denoiser* d, const Layer& L, const ConvArgs& a, int cc) {
     } else if (cc == 16) k_conv3x3<16, kConvMX, 8, 1, false><<<grid, 256, 0, d->stream>>>(a);
     else if (!a.up0) {
         // 32 output channels per block: two blocks per CU (78 KB of LDS each); more than two
-        // tiles for each: the persistent form, a tile per block again until each would get
-        // three (fewer, longer blocks leave too many idle at the end). 540 tiles and groups
-        // on 512 resident blocks: 16.9 us without, 17.6 us with it; 1530: 26.2 and 25.8 us.
+        // tiles and channel groups for each: the persistent form with the resident blocks over
+        // equal ranges. Kernel times (us) tile per block (k_conv_dma) / persistent, 64 -> 96 and
+        // 96 -> 96 channels: 1.1 times the resident blocks 13.0 / 14.0 and 17.5 / 19.7, 1.5 times
+        // 14.9 / 15.2 and 19.7 / 20.6, 2.0 times (342 tiles) 20.8 / 19.5 and 28.8 / 28.8, 3.0
+        // times (510) 26.2 / 20.0 and 36.3 / 28.3, 5.6 times (960) 44.3 / 36.4 and 61.1 / 49.4.
+        // Persistent with a tile per block lies between them (24.2 and 32.3 at 510), also where
+        // equal ranges leave blocks idle (512 tiles: four each on 384 of 512 blocks, 23.0 and
+        // 33.9; a tile per block 24.7 and 33.2).
         ConvArgs p = a;
         p.tiles_x = (int)cdiv(a.W, 16);
         p.tiles_y = (int)cdiv(a.H, 16);
@@ -1945,7 +1950,7 @@ void launch_conv(ohpt_denoiser* d, const Layer& L, const ConvArgs& a, int cc) {
             if (a.mask0) k_conv_dma<true><<<grid, 512, 0, d->stream>>>(a);
             else k_conv_dma<false><<<grid, 512, 0, d->stream>>>(a);
         } else {
-            p.per_block = work < 3 * slots - ncout ? 1 : (int)cdiv(n_tiles, (uint64_t)std::max<int64_t>(1, slots / ncout));
+            p.per_block = (int)cdiv(n_tiles, (uint64_t)std::max<int64_t>(1, slots / ncout));
             k_conv_ring<<<(cdiv(n_tiles, p.per_block) * ncout + 7u) & ~7u, 512, 0, d->stream>>>(p);
         }
     }

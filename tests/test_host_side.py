@@ -174,3 +174,30 @@ print(*held(8, 8, 3 * 2048), *held(4800, 4800, 24 << 20))
     scene, texture, large_scene, large_texture = map(int, out.split())
     assert abs(large_scene - scene) < (1 << 20), (scene, large_scene)
     assert abs(large_texture - texture) < (1 << 20), (texture, large_texture)
+
+
+@pytest.mark.parametrize("h,w", [(1080, 1920), (1088, 1936), (736, 1024), (512, 768)])
+def test_persistent_convolutions_fit_the_resident_blocks(recorded, h, w):
+    """Two blocks per compute unit are resident: layers of at most twice as many tiles and channel
+    groups run one block for each, larger ones as many blocks as are resident, which walk equal ranges."""
+    out = recorded(f"""
+d = ohpt.Denoiser(seed=1)
+R.rec_clear_launches()
+d.infer(np.zeros((1, {h}, {w}, 4), np.float32))
+for name, g in launches():
+    if "k_conv_ring" in name or "k_conv_dma" in name:
+        print("ring" if "k_conv_ring" in name else "dma", *g)
+""")
+    got = [line.split() for line in out.strip().split("\n")]
+    # level and groups of 32 output channels of the layers without an upsampled or feature input
+    layers = [(1, 2), (1, 2), (2, 3), (2, 3), (3, 4), (3, 4), (4, 5), (4, 5), (3, 4), (2, 3), (1, 2)]
+    up = lambda a, b: -(-a // b)
+    assert len(got) == len(layers)
+    for (level, groups), (kind, *grid) in zip(layers, got):
+        x, y = up(up(w, 16) * 16 >> level, 16), up(up(h, 16) * 16 >> level, 16)
+        if x * y * groups <= 2 * 512:
+            assert (kind, list(map(int, grid))) == ("dma", [x, y, groups])
+        else:
+            ranges = up(x * y, up(x * y, 512 // groups))
+            assert (kind, int(grid[0])) == ("ring", up(ranges * groups, 8) * 8)
+            assert ranges * groups <= 512
