@@ -94,14 +94,10 @@ size_t trace_overflow_bytes();
 void launch_extend(const DevScene& S, const uint32_t* queue, const uint32_t* count, uint32_t max_count,
                    const float4* ray_o, const float4* ray_d, float4* hits, uint32_t* fetch, uint32_t* ovf,
                    unsigned long long* stats, hipStream_t s, uint32_t max_blocks = 0);
-// Shadow rays: sh_o[j] = (o, tmax), sh_d[j] = (d, pid*2+k bits), sh_c[j] = contribution;
-// unoccluded ones add sh_c into ln[k][pid] and, when `vis` is given, set bit
-// 2*bounce+k of vis[pid] (for path replay).
-void launch_connect(const DevScene& S, const uint32_t* count, uint32_t max_count, const float4* sh_o,
-                    const float4* sh_d, const float4* sh_c, float4* ln0, float4* ln1, uint32_t* fetch,
-                    uint32_t* ovf, uint32_t* vis, uint32_t bounce, hipStream_t s);
-// One launch for the extension rays of bounce b+1 (closest hit, into `hits`)
-// and the shadow rays of bounce b (any hit, as launch_connect).
+// One launch for the extension rays of bounce b+1 (closest hit, into `hits`) and the
+// shadow rays of bounce b (any hit): sh_o[j] = (o, tmax), sh_d[j] = (d, pid*2+k bits),
+// sh_c[j] = contribution; unoccluded ones add sh_c into ln[k][pid] and, when `vis` is
+// given, set bit 2*bounce+k of vis[pid] (for path replay).
 void launch_extend_connect(const DevScene& S, const uint32_t* queue, const uint32_t* count_ext, uint32_t max_ext,
                            const float4* ray_o, const float4* ray_d, float4* hits, const uint32_t* count_sh,
                            uint32_t max_sh, const float4* sh_o, const float4* sh_d, const float4* sh_c, float4* ln0,

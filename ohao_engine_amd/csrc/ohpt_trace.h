@@ -111,8 +111,7 @@ __device__ __forceinline__ bool tri_hit(const RayPre& r, float4 a, float4 b, flo
 
 // Child order key: the entry distance's bits mapped to an unsigned total
 // order, the two low bits replaced by the slot (keys of one node are distinct;
-// entries within four ulps order by slot). A missed child (+inf) sorts last.
-constexpr uint32_t kKeyMiss = 0xFF800000u;
+// entries within four ulps order by slot).
 __device__ __forceinline__ uint32_t order_key(float e, uint32_t slot) {
     const uint32_t b = __float_as_uint(e);
     const uint32_t m = (b & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u;

@@ -403,14 +403,6 @@ __global__ __launch_bounds__(kTraceBlock) void k_extend(DevScene S, ExtendIO io,
     persistent_trace<0, kStats>(S, io, *count, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf, stats);
 }
 
-__global__ __launch_bounds__(kTraceBlock) void k_connect(DevScene S, ConnectIO io, const uint32_t* __restrict__ count,
-                                                         uint32_t* __restrict__ fetch, uint32_t* __restrict__ ovf) {
-    __shared__ uint32_t lds[kStackLds * kTraceBlock];
-    __shared__ uint2 pend[kPend * kTraceBlock];
-    const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x;
-    persistent_trace<1, false>(S, io, *count, fetch, lds + threadIdx.x, pend + threadIdx.x, ovf + (size_t)g * kStackOvf, nullptr);
-}
-
 template <bool kStats>
 __global__ __launch_bounds__(kTraceBlock) void k_extend_connect(DevScene S, FusedIO io,
                                                                 const uint32_t* __restrict__ count_ext,
@@ -477,15 +469,6 @@ void launch_extend(const DevScene& S, const uint32_t* queue, const uint32_t* cou
     if (max_blocks) grid = std::min(grid, max_blocks);
     if (stats) k_extend<true><<<grid, kTraceBlock, 0, s>>>(S, io, count, fetch, ovf, stats);
     else k_extend<false><<<grid, kTraceBlock, 0, s>>>(S, io, count, fetch, ovf, nullptr);
-}
-
-void launch_connect(const DevScene& S, const uint32_t* count, uint32_t max_count, const float4* sh_o,
-                    const float4* sh_d, const float4* sh_c, float4* ln0, float4* ln1, uint32_t* fetch,
-                    uint32_t* ovf, uint32_t* vis, uint32_t bounce, hipStream_t s) {
-    if (max_count == 0) return;
-    ConnectIO io{sh_o, sh_d, sh_c, ln0, ln1, vis, bounce};
-    const uint32_t grid = std::min(trace_grid_blocks(), (max_count + kTraceBlock - 1) / kTraceBlock);
-    k_connect<<<grid, kTraceBlock, 0, s>>>(S, io, count, fetch, ovf);
 }
 
 void launch_extend_connect(const DevScene& S, const uint32_t* queue, const uint32_t* count_ext, uint32_t max_ext,
