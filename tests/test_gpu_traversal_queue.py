@@ -2,6 +2,9 @@
 bit for bit: triangles that all overlap (four leaf hits in one node, a stack deeper
 than its LDS part), origins on box planes, distances from below zero, and ray
 counts around the blocks, the resident threads and the 64 fetch groups."""
+import re
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -77,3 +80,38 @@ def test_ray_counts(oracle, n):
     sc = S.displaced_sphere(6, 0.2, 1)
     V, F = sc[0], sc[3]
     check(oracle, V[F.reshape(-1)].reshape(-1, 9), rays_in(-1.2, 1.2, n, n))
+
+
+def stack_depth(nodes, ray, t_hit):
+    """Entries on the stack where `ray` needs most, with every box behind its hit culled from
+    the start: any traversal in this order holds these, and more while its hit is farther."""
+    box = nodes[:, :24].view(np.float32).astype(np.float64).reshape(-1, 2, 3, 4)
+    origin, d = ray[0:3].astype(np.float64), ray[4:7].astype(np.float64)
+    inv = 1.0 / np.where(np.abs(d) < 1e-20, 1e-20, d)
+    stack, deepest = [0], 0
+    while stack:
+        n = stack.pop()
+        t = (box[n] - origin[:, None]) * inv[:, None]
+        near = np.maximum(np.minimum(t[0], t[1]).max(0), ray[3])
+        far = np.minimum(np.maximum(t[0], t[1]).min(0), t_hit * (1 - 1e-6))
+        stack += [int(nodes[n, 24 + k]) for k in np.argsort(-near)
+                  if near[k] <= far[k] and nodes[n, 24 + k] < 0x80000000]
+        deepest = max(deepest, len(stack))
+    return deepest
+
+
+def test_stack_deeper_than_its_lds_part(oracle):
+    """The rays with most visits of the 20,000 overlapping triangles spill to global memory."""
+    header = Path(ohpt.__file__).parent / "csrc" / "ohpt_internal.h"
+    lds = int(re.search(r"#define OHPT_STACK_LDS (\d+)", header.read_text()).group(1))
+    pos, rays = overlapping(20000, 20000), rays_in(-0.5, 1.5, 3000, 20000)
+    visits = check(oracle, pos, rays)
+    rays = rays[np.argsort(-visits.astype(np.int64))[:20]]
+    ctx = ohpt.Context(32, 32)
+    ctx.load_scene(scene(pos))
+    hits, nodes = ctx.trace_rays(rays), ctx.export_bvh4()
+    ctx.close()
+    t = np.where(hits[:, 1].view(np.uint32) == 0xFFFFFFFF, np.inf, hits[:, 0])
+    depths = [stack_depth(nodes, r, v) for r, v in zip(rays, t)]
+    print(f"stack depths {sorted(depths)} with {lds} entries in LDS", flush=True)
+    assert sum(d > lds for d in depths) >= 10
