@@ -24,10 +24,11 @@
 // Bounded by the vector pipe and the return of divergent node loads together (each
 // 60-70 % busy on 10^6 incoherent rays), and by the longest rays at the end of a
 // launch. Against one triangle test per leaf in the step, a sorting network with
-// selects, and one fetch counter: 10^6 rays on the 3.1M-triangle scene 541 -> 508 us,
-// its 1920x1080 frame 3.04 -> 2.74 ms, the reference estimator's frame on 2058
-// triangles 4.32 -> 3.08 ms (nearly all of it the counters'), 512x512 turntable
-// 2.41 -> 2.33 ms.
+// selects, refills below 16 lanes and one fetch counter (both builds in turn in one run,
+// passes in a row, which is how every time in this file is taken): 1920x1080 frame of the
+// 3.1M-triangle scene 3.11 -> 2.83 ms, the reference estimator's frame on 2058
+// triangles 4.69 -> 3.44 ms, 512x512 turntable 2.44 -> 2.34 ms. The reference frame varies
+// between runs, 3.4 to 3.7 ms with what the process measured before it.
 //
 // The ray/box and ray/triangle tests and the child order key are in ohpt_trace.h.
 #pragma clang fp contract(off)
@@ -218,7 +219,9 @@ __device__ __forceinline__ void persistent_trace(const DevScene& S, const IO& io
     // fewer rays than resident threads never touch the counters). The rays beyond
     // are dealt in runs of 64 to `groups` groups of blocks, each with a counter of its
     // own in its own cache line: with one counter every wave's additions queued at one
-    // address (the reference estimator's 1080p frame 4.36 ms, 3.08 ms with 64).
+    // address (one counter / 64 with all else alike: the reference estimator's 1080p frame
+    // 5.09 / 3.39 ms, the 3.1M-triangle frame 2.98 / 2.84 ms, its 10^6 rays 615 / 505 us,
+    // turntable 2.44 / 2.33 ms).
     const uint32_t nthreads = gridDim.x * blockDim.x;
     bool drained = nthreads >= count;
     const uint32_t groups = min(kFetchGroups, gridDim.x), group = blockIdx.x % groups;
