@@ -361,8 +361,6 @@ def main():
         for k in acc:
             acc[k] += getattr(st, k)
     rays = acc["rays_extend"] + acc["rays_shadow"]
-    byts = trace_bytes(rays, acc["node_visits"], acc["tri_tests"])
-    achieved = byts / (acc["ms_extend"] * 1e-3) / 1e9 if acc["ms_extend"] > 0 else 0.0
     traffic, pmc = None, {}
     if TRAFFIC_FILE.exists():
         try:
@@ -370,6 +368,11 @@ def main():
             traffic = pmc.get("bytes_per_launch")
         except Exception:
             traffic, pmc = None, {}
+    # the kernels visit a few nodes that a sequential traversal culls (a hit whose leaf is
+    # still queued does not cull yet): those are not counted as necessary bytes
+    needed = min(float(acc["node_visits"]), pmc.get("sequential_node_visits_per_ray", float("inf")) * rays)
+    byts = trace_bytes(rays, needed, acc["tri_tests"])
+    achieved = byts / (acc["ms_extend"] * 1e-3) / 1e9 if acc["ms_extend"] > 0 else 0.0
     roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                 "kernel": "LBVH traversal: k_extend (bounce 0) + k_extend_connect (closest-hit rays of bounce b+1 "
@@ -378,6 +381,7 @@ def main():
                 "avg_launch_ms": round(acc["ms_extend"] / max(acc["extend_launches"], 1), 5),
                 "algorithmic_bytes_per_launch": round(byts / max(acc["extend_launches"], 1)),
                 "node_visits_per_ray": round(acc["node_visits"] / max(rays, 1), 3),
+                "sequential_node_visits_per_ray": pmc.get("sequential_node_visits_per_ray"),
                 "tri_tests_per_ray": round(acc["tri_tests"] / max(rays, 1), 3),
                 "profiled_frames": prof_steps, "profiled_ms_per_frame": round(acc["ms_total"] / prof_steps, 4),
                 "l2_hit_pct": pmc.get("l2_hit_pct"), "occupancy_pct_first_bounce": pmc.get("occupancy_pct_first_bounce"),

@@ -21,8 +21,8 @@
 // what the late hit lets through meanwhile is dropped too. Every FP operation
 // matches the sequential restatement in the oracle, and hits agree bit for bit.
 //
-// Bounded by the vector pipe and the return of divergent node loads together (each
-// 60-70 % busy on 10^6 incoherent rays), and by the longest rays at the end of a
+// Bounded by the return of divergent node loads and the vector pipe together (64 % and
+// 53 % busy on 10^6 incoherent rays), and by the longest rays at the end of a
 // launch. Against one triangle test per leaf in the step, a sorting network with
 // selects, refills below 16 lanes and one fetch counter (both builds in turn in one run,
 // passes in a row, which is how every time in this file is taken): 1920x1080 frame of the
