@@ -796,9 +796,9 @@ __global__ __launch_bounds__(512) void k_conv_dma(ConvArgs a) {
 // the weights stay in LDS; halo addresses are kept per lane, border checks only where
 // a tile has a border. Bounded by the latency of the halo loads (two blocks per CU,
 // 78 KB each) and the LDS reads. 1920x1080 with / without: 32 -> 64 channels at half
-// size 34 / 43 us, 64 -> 64 52 / 64 us (740 TFLOP/s), 96 -> 96 at a quarter 35 / 36 us.
-// Below two tiles and channel groups per resident block its longer prologue costs
-// 0.5-1 us a layer, and k_conv_dma runs.
+// size 34 / 43 us, 64 -> 64 47 / 63 us (817 TFLOP/s), 96 -> 96 at a quarter 28 / 36 us.
+// Where a block gets one tile its longer prologue costs 0.5-1.5 us a layer; launch_conv
+// says from where on it runs.
 __global__ __launch_bounds__(512, 4) void k_conv_ring(ConvArgs a) {
     constexpr int CC = 32, RW = 16, TX = 16, NO = 32, KS = 9;
     constexpr int HX = TX + 2, HP = HX * (RW + 2);   // 18 x 18 halo pixels
