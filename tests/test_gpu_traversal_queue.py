@@ -1,7 +1,9 @@
 """The traversal's leaf queue, stack and ray dealing against the sequential oracle,
 bit for bit: triangles that all overlap (four leaf hits in one node, a stack deeper
 than its LDS part), origins on box planes, distances from below zero, and ray
-counts around the blocks, the resident threads and the 64 fetch groups."""
+counts around the blocks, the resident threads and the 64 fetch groups. Batches that
+are resident at once take the kernel with a ray per thread, larger ones the
+persistent one with the queue: each scene goes through both."""
 import re
 from pathlib import Path
 
@@ -37,17 +39,23 @@ def rays_in(lo, hi, n, seed, tmin=0.0, tmax=np.inf):
     return r
 
 
+RESIDENT = 327680   # threads of a 256-CU grid
+
+
 def check(oracle, pos, rays):
     sc = scene(pos)
-    ctx = ohpt.Context(32, 32)
-    ctx.load_scene(sc)
-    got = ctx.trace_rays(rays)
-    occ = ctx.occluded_rays(rays)
-    ctx.close()
     o = oracle.OracleScene(sc)
     want, visits, _ = o.trace(rays)
-    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
-    assert np.array_equal(occ, o.occluded(rays))
+    occluded = o.occluded(rays)
+    ctx = ohpt.Context(32, 32)
+    ctx.load_scene(sc)
+    # once as they are, and over and over in another order until they are more than are resident
+    order = np.concatenate([np.random.default_rng(k).permutation(len(rays)) for k in range(RESIDENT // len(rays) + 1)])
+    for batch in (np.arange(len(rays)), order[:RESIDENT + 1001] if len(rays) > 1 else order[:0]):
+        if len(batch):
+            assert np.array_equal(ctx.trace_rays(rays[batch]).view(np.uint32), want[batch].view(np.uint32))
+            assert np.array_equal(ctx.occluded_rays(rays[batch]), occluded[batch])
+    ctx.close()
     return visits
 
 
@@ -73,7 +81,7 @@ def test_origins_on_box_planes(oracle):
     check(oracle, pos, rays)
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 129, 327679, 327681, 327680 + 64 * 64 + 1, 700001])
+@pytest.mark.parametrize("n", [1, 63, 64, 129, 327679, 327680, 327681, 327680 + 64 * 64 + 1, 700001])
 def test_ray_counts(oracle, n):
     """A 256-CU grid holds 327,680 threads; further rays are dealt in 64 groups."""
     print(f"count {n}", flush=True)
@@ -114,4 +122,4 @@ def test_stack_deeper_than_its_lds_part(oracle):
     t = np.where(hits[:, 1].view(np.uint32) == 0xFFFFFFFF, np.inf, hits[:, 0])
     depths = [stack_depth(nodes, r, v) for r, v in zip(rays, t)]
     print(f"stack depths {sorted(depths)} with {lds} entries in LDS", flush=True)
-    assert sum(d > lds for d in depths) >= 10
+    assert sum(d - 1 > lds for d in depths) >= 10   # the nearest child may be kept in a register
