@@ -93,7 +93,7 @@ def padded(a):
     return out
 
 
-@pytest.mark.parametrize("w,h", [(17, 3), (257, 513)])
+@pytest.mark.parametrize("w,h", [(17, 3), (64, 64), (241, 17), (257, 513)])   # up to 4096 texels packed on the host
 @pytest.mark.parametrize("channels", [1, 2, 3, 4])
 def test_packed_texels_are_the_callers(oracle, w, h, channels):
     rng = np.random.default_rng(w + channels)
@@ -147,7 +147,7 @@ def test_unpacked_gradients_are_the_four_channel_ones(channels):
         assert np.array_equal(got, four[..., :channels])
 
 
-@pytest.mark.parametrize("w,h", [(61, 130), (512, 256), (513, 256), (700, 411)])
+@pytest.mark.parametrize("w,h", [(61, 30), (128, 64), (61, 139), (512, 256), (513, 256), (700, 411)])
 @pytest.mark.parametrize("channels", [1, 2, 3, 4])
 def test_mean_of_an_emissive_texture_chooses_between_two_emitters(oracle, w, h, channels):
     """The mean is half of the choice between the lamp and a textured emitter: with another

@@ -74,21 +74,20 @@ def test_a_failed_texture_upload_leaves_no_copy_in_flight(recorded):
     """The texels are the caller's, who may free them as soon as the call returns."""
     out = recorded("""
 failed, left = 0, []
-for update in (False, True):
-    for n in range(10):
-        ctx = ohpt.Context(16, 16)
-        t = np.ones((5, 7, 3), np.float32)
-        if update:
-            ctx.upload_texture(t)
-        R.rec_fail_copy(n)
-        try:
-            ctx.update_texture(0, t) if update else ctx.upload_texture(t)
-        except ohpt.OhptError:
-            failed += 1
-            if R.rec_pending():
-                left.append((update, n, R.rec_pending()))
-        R.rec_fail_copy(-1)
-        ctx.close()
+for update, n in [(u, k) for u in (False, True) for k in range(20)]:
+    ctx = ohpt.Context(16, 16)
+    t = np.ones((5, 7, 3) if n < 10 else (90, 100, 3), np.float32)   # packed on the host, on the device
+    if update:
+        ctx.upload_texture(t)
+    R.rec_fail_copy(n % 10)
+    try:
+        ctx.update_texture(0, t) if update else ctx.upload_texture(t)
+    except ohpt.OhptError:
+        failed += 1
+        if R.rec_pending():
+            left.append((update, n, R.rec_pending()))
+    R.rec_fail_copy(-1)
+    ctx.close()
 print(failed, left)
 """)
     failures, left = out.strip().split(" ", 1)
@@ -201,3 +200,17 @@ for name, g in launches():
             ranges = up(x * y, up(x * y, 512 // groups))
             assert (kind, int(grid[0])) == ("ring", up(ranges * groups, 8) * 8)
             assert ranges * groups <= 512
+
+
+def test_small_textures_launch_nothing(recorded):
+    """Up to 8192 texels an update is one copy: the kernels' launches take longer than the loop."""
+    out = recorded("""
+for w in (1, 8192, 8193):
+    ctx = ohpt.Context(16, 16)
+    t = np.zeros((1, w, 3), np.float32)
+    ctx.upload_texture(t)
+    R.rec_clear_launches()
+    ctx.update_texture(0, t)
+    print(R.rec_launches())
+""")
+    assert out.split() == ["0", "0", "2"]
