@@ -669,17 +669,25 @@ struct MeshRun {
     std::vector<float> pos, nrm, uv;
 };
 
-void expand_mesh(const ohpt_context* c, const ohpt_context::MeshRec& m, MeshRun& r) {
-    const MeshTransform x = mesh_transform(m);
-    float P[9], Nn[9];
-    for (uint32_t t = 0; t < m.nt; ++t) {
-        world_triangle(m, x, t, c->any_nrm, P, Nn);
-        r.pos.insert(r.pos.end(), P, P + 9);
-        if (c->any_nrm) r.nrm.insert(r.nrm.end(), Nn, Nn + 9);
-        for (int k = 0; c->any_uv && k < 3; ++k) {
-            const float* u = m.uv.empty() ? nullptr : &m.uv[(size_t)m.idx[(size_t)t * 3 + k] * 2];
-            r.uv.push_back(u ? u[0] : 0.0f);
-            r.uv.push_back(u ? u[1] : 0.0f);
+// Meshes [begin, end), which follow one another in the scene, into r.
+void expand_meshes(const ohpt_context* c, size_t begin, size_t end, MeshRun& r) {
+    size_t n = 0;
+    for (size_t i = begin; i < end; ++i) n += c->meshes[i].nt;
+    r.base = c->meshes[begin].base;
+    r.pos.resize(n * 9);
+    if (c->any_nrm) r.nrm.resize(n * 9);
+    if (c->any_uv) r.uv.resize(n * 6);
+    float *P = r.pos.data(), *N = r.nrm.data(), *U = r.uv.data();
+    for (size_t i = begin; i < end; ++i) {
+        const ohpt_context::MeshRec& m = c->meshes[i];
+        const MeshTransform x = mesh_transform(m);
+        for (uint32_t t = 0; t < m.nt; ++t, P += 9) {
+            world_triangle(m, x, t, c->any_nrm, P, N);
+            if (c->any_nrm) N += 9;
+            if (!c->any_uv) continue;
+            for (int k = 0; !m.uv.empty() && k < 3; ++k)
+                std::memcpy(U + 2 * k, &m.uv[(size_t)m.idx[(size_t)t * 3 + k] * 2], 8);
+            U += 6;
         }
     }
 }
@@ -828,10 +836,10 @@ int ohpt_scene_commit(ohpt_context* c) {
             if (int r = place_mesh(c, c->meshes[i++], staged)) return r;
             continue;
         }
-        MeshRun& run = runs.emplace_back();
-        run.base = c->meshes[i].base;
-        for (; i < c->meshes.size() && c->meshes[i].nt < kHostMeshTriangles; ++i) expand_mesh(c, c->meshes[i], run);
-        if (int r = place_run(c, run)) return r;
+        const size_t begin = i;
+        while (i < c->meshes.size() && c->meshes[i].nt < kHostMeshTriangles) ++i;
+        expand_meshes(c, begin, i, runs.emplace_back());
+        if (int r = place_run(c, runs.back())) return r;
     }
     const uint32_t ni = n > 1 ? n - 1 : 1;
     HIPCHK(c->d_nodes.ensure((size_t)ni * 64));
