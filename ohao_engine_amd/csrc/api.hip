@@ -1011,7 +1011,7 @@ namespace {
 // back take longer than the loop. Update in us, on the device / here: from the host 1 texel
 // 32 / 16, 8192 of three channels 38 / 20, of four 39 / 34; from the device 1 texel 40 / 27,
 // 4096 of three channels 39 / 25, of four 39 / 34.
-constexpr size_t kHostTexels = 8192, kHostTexelsOnDevice = 4096;
+constexpr size_t kHostTexels = 8192, kHostTexelsOnDevice = 4096, kHostGradientTexels = 10240;
 int fill_small_texture(ohpt_context* c, TexStore& t, const float* texels, int on_device) {
     const size_t n = (size_t)t.w * t.h, stride = t.c >= 2 ? 4 : 1;
     std::vector<float> source, packed(n * stride, 0.0f);
@@ -1558,7 +1558,18 @@ int ohpt_read_texture_gradient(ohpt_context* c, int32_t id, float* out, int on_d
     HIPCHK(enter(c));
     const size_t n = (size_t)t.w * t.h, bytes = n * t.c * 4;
     const float* src = c->grad_arena.as<float>() + c->grad_off[(size_t)id];
-    if (t.c == 2 || t.c == 3) {
+    const bool padded = t.c == 2 || t.c == 3;
+    if (padded && !on_device && n <= kHostGradientTexels) {
+        // fewer texels than a launch is worth: 64x64 of three channels 26 us unpacked on the
+        // device, 17 here, 129x64 28 and 25; 128x128 32 and 40
+        std::vector<float> packed(n * 4);
+        HIPCHK(hipMemcpyAsync(packed.data(), src, n * 16, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (size_t i = 0; i < n; ++i)
+            for (uint32_t k = 0; k < t.c; ++k) out[i * t.c + k] = packed[i * 4 + k];
+        return OHPT_OK;
+    }
+    if (padded) {
         HIPCHK(c->tmp.ensure(bytes));
         launch_texel_unpack(src, n, t.c, c->tmp.as<float>(), c->stream);
         HIPCHK(hipGetLastError());

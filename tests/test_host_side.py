@@ -214,3 +214,18 @@ for w in (1, 8192, 8193):
     print(R.rec_launches())
 """)
     assert out.split() == ["0", "0", "2"]
+
+
+def test_small_gradients_launch_nothing(recorded):
+    out = recorded("""
+import dataclasses
+for w in (1, 10240, 10241):
+    sc = dataclasses.replace(S.lantern(freq=2, tex_size=64), textures=[np.zeros((1, w, 3), np.float32)], width=16, height=16)
+    ctx = ohpt.Context(16, 16)
+    ctx.load_scene(sc)
+    ctx.adjoint(np.ones((16, 16, 4), np.float32), 1)
+    R.rec_clear_launches()
+    ctx.texture_gradient(0, (1, w, 3))
+    print(R.rec_launches())
+""")
+    assert out.split() == ["0", "0", "1"]
