@@ -338,8 +338,9 @@ int ohpt_occluded_rays(ohpt_context* ctx, const float* rays, uint32_t* out, uint
  * are device pointers on the context's device (16-byte aligned, same layouts
  * as ohpt_trace_rays); results equal ohpt_trace_rays's bit for bit. The
  * traversal's fetch counter and stack-overflow slots live in one fixed array
- * per device (36 MiB + 8 KiB, held until the process ends), cleared by a
- * kernel at each call. The call only enqueues work on the context's stream
+ * per device (36 MiB + 8 KiB, held until the process ends), the counters
+ * cleared by a kernel at each call of more than 131,072 rays (fewer need
+ * none). The call only enqueues work on the context's stream
  * (ohpt_synchronize before reading hits on the host). Calls that overlap on
  * one device — from any contexts or threads — race on that array and must be
  * serialised by the caller. n above 2^31 is rejected (OHPT_ERR_INVALID_ARG). */
